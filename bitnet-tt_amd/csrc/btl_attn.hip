@@ -9,11 +9,13 @@
 // caches [B, Hkv, S, D] bf16 (the reference's KV-cache shape); output
 // [B, H D] bf16 (heads concatenated, o_proj's input).  D = 128.
 //
-// One workgroup of 8 waves per (user, key-value head).  Measured on MI355X,
-// splitting the context over more workgroups (to use all 256 CUs) and
-// merging their partials through the workspace was slower at the 2B shape:
-// the merge's store-acknowledge-count-reload chain costs more than the extra
-// CUs gain.
+// One workgroup of 8 waves per (user, key-value head), or, where the pairs
+// leave most of the chip idle, one per split of a pair's context
+// (btl_attn_body.h): each split publishes its partial with coherent stores and
+// counts itself, and the last of a pair to arrive merges them in split order.
+// Nothing waits on another workgroup.  (At the 2B shape's 160 pairs and 512
+// positions the store-acknowledge-count-reload chain costs more than the
+// extra CUs gain: one split.)
 #include <hip/hip_runtime.h>
 
 #include "btl.h"
@@ -36,10 +38,54 @@ struct AttnArgs {
   int B, H, Hkv, G, S;
   float scale;
   int adjacent;            // 1: RoPE pairs (2i, 2i+1); 0: (i, i + D/2)
+  int smax;                // workgroups per (user, key-value head)
+  uint32_t* count;         // [pairs] splits arrived (zero between calls)
+  float* part;             // [pairs][smax][kAtPartFloats]
 };
 
+// Workspace: the error word, then (smax > 1) the arrival counters and partials.
+constexpr int64_t kAttnCount = 256;
+constexpr int64_t kAttnPart = kAttnCount + kAtSplitItems * 4;
+static_assert(kAttnPart % 16 == 0, "partials aligned");
+
+// Publishes this split's partial; true in the workgroup that arrived last,
+// with every split's partial in Ms, Ls, Os.
+__device__ bool attn_gather(const AttnArgs& p, const AttnPair& a, int pair, int n, const AttnPartial& mine,
+                            int* s_last, float (&Ms)[kAtMaxSplits], float (&Ls)[kAtMaxSplits],
+                            float (&Os)[kAtMaxSplits]) {
+  const int tid = threadIdx.x, g = tid / kAtD;
+  float* const base = p.part + (int64_t)pair * p.smax * kAtPartFloats;
+  if (g < a.G) {
+    float* const o = base + a.split * kAtPartFloats;
+    st_coherent(o + tid, mine.O);
+    if (tid % kAtD == 0) {
+      st_coherent(o + kAtMaxG * kAtD + 2 * g, mine.M);
+      st_coherent(o + kAtMaxG * kAtD + 2 * g + 1, mine.L);
+    }
+  }
+  wait_memory();
+  __syncthreads();  // the whole partial is out before the arrival is counted
+  if (tid == 0) *s_last = atomicAdd(p.count + pair, 1u) == (unsigned)(n - 1);
+  __syncthreads();
+  if (!*s_last) return false;
+  if (tid == 0) st_coherent(p.count + pair, 0u);  // left clean for the next call
+  const int gc = min(g, a.G - 1);
+#pragma unroll
+  for (int i = 0; i < kAtMaxSplits; ++i)
+    if (i < n) {
+      const float* const o = base + i * kAtPartFloats;
+      Os[i] = ld_coherent(o + tid);
+      Ms[i] = ld_coherent(o + kAtMaxG * kAtD + 2 * gc);
+      Ls[i] = ld_coherent(o + kAtMaxG * kAtD + 2 * gc + 1);
+    }
+  return true;
+}
+
+// SPLIT: smax > 1 workgroups per pair.
+template <bool SPLIT>
 __global__ __launch_bounds__(64 * kAtWaves, 1) void k_decode_attention(AttnArgs p) {
   __shared__ __attribute__((aligned(16))) AttnSmem s;
+  __shared__ int s_last;
   const int tid = threadIdx.x;
   BTL_TRACE_AT(0);
   AttnPair a;
@@ -50,16 +96,23 @@ __global__ __launch_bounds__(64 * kAtWaves, 1) void k_decode_attention(AttnArgs 
   a.Hkv = p.Hkv;
   a.G = p.G;
   a.S = p.S;
-  a.hk = blockIdx.x % p.Hkv;
-  a.b = blockIdx.x / p.Hkv;
-  a.pos = p.pos[a.b];
+  // every pair's split 0 first: they are spread over the XCDs, and where a
+  // context is one round they do not queue behind workgroups that only leave
+  const int pairs = p.B * p.Hkv;
+  const int pair = SPLIT ? blockIdx.x % pairs : blockIdx.x;
+  a.smax = SPLIT ? p.smax : 1;
+  a.split = SPLIT ? blockIdx.x / pairs : 0;
+  a.hk = pair % p.Hkv;
+  a.b = pair / p.Hkv;
+  a.pos = __builtin_amdgcn_readfirstlane(p.pos[a.b]);
   a.scale = p.scale;
   a.adjacent = p.adjacent;
   a.tid = tid;
-  if (!a.pos_ok() && tid == 0 && a.hk == 0) st_coherent(p.error, 1);
+  if (a.split != 0 && a.split >= a.splits()) return;
   AttnRound r;
-  att_load_round(a, 0, r);
+  att_load_first(a, r);
   BTL_TRACE_AT(1);
+  if (!a.pos_ok() && tid == 0 && a.hk == 0 && a.split == 0) st_coherent(p.error, 1);
   // the new token's rows of the group: q rows hk G .. hk G + G - 1, k row hk, v row hk
   const uint16_t* qrow = p.qkv + (int64_t)a.b * p.ldq;
   if (tid < (kAtMaxG + 2) * (kAtD / 8)) {
@@ -70,7 +123,14 @@ __global__ __launch_bounds__(64 * kAtWaves, 1) void k_decode_attention(AttnArgs 
   }
   __syncthreads();
   BTL_TRACE_AT(2);
-  const uint16_t o = att_body(a, s, r, true);
+  AttnPartial part;
+  uint16_t o = att_body(a, s, r, part, true);
+  const int n = SPLIT ? a.splits() : 1;
+  if (SPLIT && n > 1) {
+    float Ms[kAtMaxSplits], Ls[kAtMaxSplits], Os[kAtMaxSplits];
+    if (!attn_gather(p, a, pair, n, part, &s_last, Ms, Ls, Os)) return;
+    o = tid < a.G * kAtD ? att_merge(s, tid, n, Ms, Ls, Os) : 0;
+  }
   if (tid < a.G * kAtD) p.out[(int64_t)a.b * p.H * kAtD + (a.hk * a.G) * kAtD + tid] = o;
   BTL_TRACE_AT(7);
 }
@@ -85,7 +145,10 @@ extern "C" {
 
 int64_t btl_decode_attention_workspace_bytes(int64_t B, int64_t H, int64_t Hkv, int64_t S) {
   if (B <= 0 || Hkv <= 0 || H <= 0 || H % Hkv || H / Hkv > kAtMaxG || S <= 0) return 0;
-  return 256;  // the error word
+  // the error word; the counters and partials of the splits, where a call of
+  // this shape has any (at most kAtSplitItems, on any device)
+  if (S <= kAtWaves * kAtPosWave || 2 * B * Hkv > kAtSplitItems) return kAttnCount;
+  return kAttnPart + (int64_t)kAtSplitItems * kAtPartFloats * 4;
 }
 
 int64_t btl_decode_attention_error_offset(int64_t B, int64_t Hkv) {
@@ -129,8 +192,14 @@ int btl_decode_attention(const uint16_t* qkv, int64_t B, int64_t H, int64_t Hkv,
   a.scale = scale;
   a.adjacent = rope_adjacent ? 1 : 0;
   a.error = reinterpret_cast<int32_t*>(workspace);
-  const dim3 grid((unsigned)(B * Hkv));
-  hipLaunchKernelGGL(k_decode_attention, grid, dim3(64 * kAtWaves), 0, (hipStream_t)stream, a);
+  a.smax = att_max_splits(B * Hkv, S, device_cus());
+  a.count = reinterpret_cast<uint32_t*>(static_cast<char*>(workspace) + kAttnCount);
+  a.part = reinterpret_cast<float*>(static_cast<char*>(workspace) + kAttnPart);
+  const dim3 grid((unsigned)(B * Hkv * a.smax));
+  if (a.smax > 1)
+    hipLaunchKernelGGL(k_decode_attention<true>, grid, dim3(64 * kAtWaves), 0, (hipStream_t)stream, a);
+  else
+    hipLaunchKernelGGL(k_decode_attention<false>, grid, dim3(64 * kAtWaves), 0, (hipStream_t)stream, a);
   return check_launch("decode attention");
 }
 

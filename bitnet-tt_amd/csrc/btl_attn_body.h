@@ -9,7 +9,18 @@
 // A round covers 512 cached positions, 64 per wave; every wave issues all of
 // its key and value loads (256 B per lane each) before computing, so a round
 // is one memory round trip (at context 512 the whole context is one round,
-// and the caller may issue it before the new token's q, k, v exist).
+// and the caller may issue it before the new token's q, k, v exist).  (Issuing
+// the next round's keys and values as soon as this one's have left their
+// registers gains 5 % at 2048 positions and more, 160 pairs, and costs 1 us at
+// 512: 64 more registers.)
+//
+// Few pairs (att_max_splits): the blocks of 64 positions of a context longer
+// than one round are split over up to 8 workgroups per pair, whose partials
+// (max, sum, unnormalised output per head) meet in one of them in a fixed
+// order.  One pair per workgroup leaves most of the chip idle there and walks
+// the rounds one after another: two users at 4096 positions, 5 key-value
+// heads, 48 us on 10 workgroups.  The number of splits depends on the pairs,
+// the cache length and the position only, so both callers give the same bits.
 //  - Scores: v_mfma_f32_16x16x32_bf16, the G rotated query rows (head g at
 //    row 4 g, the other rows zero) against 16 cached key rows per MFMA (keys
 //    contiguous along D, the contraction, so the B operands load straight
@@ -39,10 +50,32 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 constexpr int kAtD = 128;                        // head dimension
 constexpr int kAtWaves = 8;                      // waves per workgroup
 constexpr int kAtPosWave = 64;                   // positions per wave and round
-constexpr int kAtRound = kAtWaves * kAtPosWave;  // positions per round
 constexpr int kAtMaxG = 4;                       // query heads per key-value head
 constexpr int kAtVPitch = kAtD + 4;              // bf16 per LDS value row (8-byte pad)
 constexpr int kAtVRows = 32;                     // value rows of a wave staged at once
+constexpr int kAtMaxSplits = 8;                  // workgroups one pair's context is split over
+constexpr int kAtMinBlocks = 4;                  // blocks of 64 positions a split is worth
+// Workgroups that the pairs of a call are spread over: the one-launch step has
+// the CUs without its 32 row workgroups.
+constexpr int kAtSplitItems = 224;
+constexpr int kAtPartFloats = kAtMaxG * kAtD + 2 * kAtMaxG;  // one split's partial: outputs, maxima, sums
+
+// Most splits per pair: one where the pairs alone fill the chip or the cache
+// is a single round.  Measured on MI355X (20 / 5 heads, cache of 4096, one
+// workgroup a pair -> split, us a launch): 1 user at 640 / 2048 / 4096
+// positions 11.6 -> 11.0, 26.5 -> 11.4, 50.4 -> 13.6; 8 users 12.5 -> 12.0,
+// 27.8 -> 14.8, 56.4 -> 23.3; 22 users 13.1 -> 14.4, 36.2 -> 27.6, 66.3 ->
+// 47.3.  Up to 512 positions a context stays whole (10.2 us; the workgroups
+// that find nothing to do cost 0.5 us).  Eight splits and not sixteen: with
+// the words of sixteen the one-launch step's instance spills.
+inline int att_max_splits(int64_t pairs, int64_t S, int64_t cus) {
+  int64_t n = (cus - 32 < kAtSplitItems ? cus - 32 : kAtSplitItems) / pairs;
+  const int64_t blocks = (S + kAtPosWave - 1) / kAtPosWave;
+  if (blocks <= kAtWaves) return 1;
+  if (n > blocks / kAtMinBlocks) n = blocks / kAtMinBlocks;
+  if (n > kAtMaxSplits) n = kAtMaxSplits;
+  return n > 1 ? (int)n : 1;
+}
 
 struct AttnSmem {
   uint16_t in[kAtMaxG + 2][kAtD];                   // the new token's q rows, k row, v row (as produced)
@@ -64,6 +97,7 @@ struct AttnPair {
   uint16_t* kc;       // [B, Hkv, S, D]
   uint16_t* vc;
   int Hkv, G, S, b, hk, pos;
+  int smax, split;    // most splits of the pair (att_max_splits), this workgroup's
   float scale;
   int adjacent;  // 1: RoPE pairs (2i, 2i+1); 0: (i, i + D/2)
   // This thread's index in the workgroup.  A caller that runs the body inside
@@ -73,6 +107,19 @@ struct AttnPair {
   int tid;
   __device__ __forceinline__ bool pos_ok() const { return pos >= 0 && pos < S; }
   __device__ __forceinline__ int nold() const { return pos_ok() ? pos : 0; }  // cached positions [0, nold)
+  // The pair's blocks of 64 cached positions, how many a split takes, the
+  // splits that have any, and this split's range of blocks.
+  __device__ __forceinline__ int blocks() const { return (nold() + kAtPosWave - 1) / kAtPosWave; }
+  __device__ __forceinline__ int per_split() const {
+    const int nb = blocks();
+    return smax == 1 || nb <= kAtWaves ? nb : max(kAtMinBlocks, (nb + smax - 1) / smax);
+  }
+  __device__ __forceinline__ int splits() const {
+    const int nb = blocks(), per = per_split();
+    return nb == per ? 1 : (nb + per - 1) / per;
+  }
+  __device__ __forceinline__ int block0() const { return split == 0 ? 0 : split * per_split(); }
+  __device__ __forceinline__ int block1() const { return min(blocks(), block0() + per_split()); }
   __device__ __forceinline__ int64_t kv_base() const { return ((int64_t)b * Hkv + hk) * S; }
 };
 
@@ -112,7 +159,7 @@ __device__ __forceinline__ v4s lds_read_tr16(const uint16_t* p) {
       (__attribute__((address_space(3))) v4s*)(__attribute__((address_space(3))) void*)p);
 }
 
-// A wave's key and value rows of round rd: K operands (4 blocks of 16
+// A wave's key and value rows of a round: K operands (4 blocks of 16
 // positions x 4 k-steps) and value pieces (dims 8 r16 .. + 8 of row 4 t + grp).
 struct AttnRound {
   uint4 kr[4][kAtD / 32];
@@ -137,22 +184,16 @@ __device__ __forceinline__ uint4 att_ld(__amdgpu_buffer_rsrc_t r, int voff, int 
   return make_uint4(v[0], v[1], v[2], v[3]);
 }
 
-__device__ __forceinline__ void att_load_round(const AttnPair& a, int rd, AttnRound& r) {
-  const int lane = a.tid & 63, wv = __builtin_amdgcn_readfirstlane(a.tid >> 6);
-  if (rd == 0) {  // the RoPE factors of frequency tid & 63 at the position, with the first round
-    const int i = a.tid & (kAtD / 2 - 1), pc = a.pos_ok() ? a.pos : 0;
-    r.rc = a.rcos[pc * (kAtD / 2) + i];
-    r.rs = a.rsin[pc * (kAtD / 2) + i];
-  }
-  const int r16 = lane & 15, grp = lane >> 4;
-  const int base = rd * kAtRound + kAtPosWave * wv;
+// Keys and values of this wave's block `blk` of 64 positions.
+__device__ __forceinline__ void att_load_block(const AttnPair& a, int blk, AttnRound& r) {
+  const int lane = a.tid & 63, r16 = lane & 15, grp = lane >> 4, base = blk * kAtPosWave;
   const __amdgpu_buffer_rsrc_t kc = att_rows(a.kc, a), vc = att_rows(a.vc, a);
 #pragma unroll
-  for (int blk = 0; blk < 4; ++blk) {
-    const int row = min(base + 16 * blk + r16, a.S - 1);
+  for (int b4 = 0; b4 < 4; ++b4) {
+    const int row = min(base + 16 * b4 + r16, a.S - 1);
     const int off = (row * kAtD + 8 * grp) * 2;
 #pragma unroll
-    for (int ks = 0; ks < kAtD / 32; ++ks) r.kr[blk][ks] = att_ld(kc, off, 64 * ks);
+    for (int ks = 0; ks < kAtD / 32; ++ks) r.kr[b4][ks] = att_ld(kc, off, 64 * ks);
   }
 #pragma unroll
   for (int t = 0; t < 16; ++t) {
@@ -161,8 +202,31 @@ __device__ __forceinline__ void att_load_round(const AttnPair& a, int rd, AttnRo
   }
 }
 
-// Everything after the first round's loads (att_load_round(a, 0, r), issued
-// by the caller in every wave): RoPE of the group's query rows
+// The first round, then the RoPE factors of frequency tid & 63 at the
+// position.  Split 0's first blocks do not depend on the position, which may
+// itself still be on its way (waiting for it first costs 1 us a launch); in
+// the other splits a wave with no block loads none.
+__device__ __forceinline__ void att_load_first(const AttnPair& a, AttnRound& r) {
+  const int wv = __builtin_amdgcn_readfirstlane(a.tid >> 6);
+  int blk = wv;
+  bool any = true;
+  if (a.split != 0) {
+    blk += a.split * a.per_split();
+    any = blk < a.block1();
+  }
+  if (any) att_load_block(a, blk, r);
+  const int i = a.tid & (kAtD / 2 - 1), pc = a.pos_ok() ? a.pos : 0;
+  r.rc = a.rcos[pc * (kAtD / 2) + i];
+  r.rs = a.rsin[pc * (kAtD / 2) + i];
+}
+
+// A thread's share of a split's partial: head tid / D, dimension tid % D.
+struct AttnPartial {
+  float M, L, O;
+};
+
+// Everything after the first round's loads (att_load_first, issued by the
+// caller in every wave): RoPE of the group's query rows
 // and the new k row (the new rows go to LDS and to the caches), scores,
 // online softmax, probability-weighted values, merge.  s.in holds the new
 // token's rows (q rows 0..G-1, k at kAtMaxG, v at kAtMaxG + 1) and every
@@ -170,15 +234,18 @@ __device__ __forceinline__ void att_load_round(const AttnPair& a, int rd, AttnRo
 // threads tid < G D (head tid / D, dimension tid % D), the bf16 output
 // (zero for a position outside [0, S)); the other threads return 0.  Ends
 // with every LDS access of the body complete (the caller may reuse s after
-// a barrier).
+// a barrier).  Where the pair is split, part is this split's partial instead,
+// without the new position, which att_merge adds; split 0 writes the new rows
+// to the caches.
 // Measurement builds (-DBTL_TRACE) stamp events 3-6 (RoPE done, first
 // round's softmax done, its values done, merge barriers passed) when trace is set.
-__device__ __forceinline__ uint16_t att_body(const AttnPair& a, AttnSmem& s, AttnRound& r, bool trace = false) {
+__device__ __forceinline__ uint16_t att_body(const AttnPair& a, AttnSmem& s, AttnRound& r, AttnPartial& part,
+                                             bool trace = false) {
   const int tid = a.tid, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int G = a.G;
   const bool pos_ok = a.pos_ok();
   const int nold = a.nold();
-  const int nrounds = (nold + kAtRound - 1) / kAtRound;
+  const int blk1 = a.block1();
   const int64_t kvb = a.kv_base();
   const int half = kAtD / 2;
   const int r16 = lane & 15, grp = lane >> 4;
@@ -198,7 +265,7 @@ __device__ __forceinline__ uint16_t att_body(const AttnPair& a, AttnSmem& s, Att
       const uint16_t k0 = f2bf(y0), k1 = f2bf(y1);
       s.nw[0][d0] = k0;
       s.nw[0][d1] = k1;
-      if (pos_ok) {
+      if (pos_ok && a.split == 0) {
         uint16_t* dst = a.kc + (kvb + a.pos) * kAtD;
         dst[d0] = k0;
         dst[d1] = k1;
@@ -207,7 +274,7 @@ __device__ __forceinline__ uint16_t att_body(const AttnPair& a, AttnSmem& s, Att
       const int d = 2 * i;
       const uint32_t vnew = *reinterpret_cast<const uint32_t*>(&s.in[kAtMaxG + 1][d]);
       *reinterpret_cast<uint32_t*>(&s.nw[1][d]) = vnew;
-      if (pos_ok) *reinterpret_cast<uint32_t*>(a.vc + (kvb + a.pos) * kAtD + d) = vnew;
+      if (pos_ok && a.split == 0) *reinterpret_cast<uint32_t*>(a.vc + (kvb + a.pos) * kAtD + d) = vnew;
     }
   }
   lds_barrier();  // the rotated rows are in LDS (the cache-row stores need no acknowledgement)
@@ -237,10 +304,11 @@ __device__ __forceinline__ uint16_t att_body(const AttnPair& a, AttnSmem& s, Att
 #pragma unroll
   for (int m = 0; m < kAtD / 16; ++m) o[m] = (v4f){0.f, 0.f, 0.f, 0.f};
 
+  const int nrounds = (blk1 - a.block0() + kAtWaves - 1) / kAtWaves;
   for (int rd = 0; rd < nrounds; ++rd) {
-    const int base = rd * kAtRound + kAtPosWave * wv;
-    if (base >= nold) break;  // wave-uniform: nothing cached from here on
-    if (rd > 0) att_load_round(a, rd, r);
+    const int blk = a.block0() + rd * kAtWaves + wv, base = kAtPosWave * blk;
+    if (blk >= blk1) break;  // wave-uniform: nothing cached from here on
+    if (rd > 0) att_load_block(a, blk, r);
     // scores: 4 blocks of 16 positions
     v4f sc[4];
 #pragma unroll
@@ -341,7 +409,21 @@ __device__ __forceinline__ uint16_t att_body(const AttnPair& a, AttnSmem& s, Att
   uint16_t res = 0;
   {
     const int g = tid / kAtD, d = tid % kAtD;  // 512 threads: 4 heads x 128 dims
-    if (g < G) {
+    if (g < G && a.splits() > 1) {
+      float M = -__builtin_inff();
+#pragma unroll
+      for (int w = 0; w < kAtWaves; ++w) M = fmaxf(M, s.ml[w][g][0]);
+      float L = 0.0f, O = 0.0f;
+#pragma unroll
+      for (int w = 0; w < kAtWaves; ++w) {
+        const float ww = wexp(s.ml[w][g][0], M);
+        L += ww * s.ml[w][g][1];
+        O += ww * s_o[w][g][d];
+      }
+      part.M = M;
+      part.L = L;
+      part.O = O;
+    } else if (g < G) {
       const float snew = s.snew[g];
       float M = snew;
 #pragma unroll
@@ -362,6 +444,29 @@ __device__ __forceinline__ uint16_t att_body(const AttnPair& a, AttnSmem& s, Att
   __atomic_signal_fence(__ATOMIC_SEQ_CST);
   __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this thread's LDS reads are done
   return res;
+}
+
+// The bf16 output of thread (g, d) from the splits' partials, in split order,
+// and the new position (its score and value row in s).  M, L, O: n partials.
+__device__ __forceinline__ uint16_t att_merge(const AttnSmem& s, int tid, int n, const float (&Ms)[kAtMaxSplits],
+                                              const float (&Ls)[kAtMaxSplits], const float (&Os)[kAtMaxSplits]) {
+  const int g = tid / kAtD, d = tid % kAtD;
+  const float snew = s.snew[g];
+  float M = snew;
+#pragma unroll
+  for (int i = 0; i < kAtMaxSplits; ++i)
+    if (i < n) M = fmaxf(M, Ms[i]);
+  const float wn = __expf(snew - M);
+  float L = wn;
+  float O = wn * bf2f(s.nw[1][d]);
+#pragma unroll
+  for (int i = 0; i < kAtMaxSplits; ++i)
+    if (i < n) {
+      const float ww = wexp(Ms[i], M);
+      L += ww * Ls[i];
+      O += ww * Os[i];
+    }
+  return f2bf(O * (1.0f / L));
 }
 
 }  // namespace btl

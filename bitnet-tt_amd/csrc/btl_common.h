@@ -48,6 +48,7 @@ int check_launch(const char* what);
 // CUs the stream may use.
 int coresident_check(const char* who, int64_t grid, int64_t per_cu, int64_t cus);
 int stream_cus(hipStream_t s);
+int device_cus();  // of the current device, cached (256 where there is none)
 int kernel_per_cu(const void* kernel, int threads);
 int check_coresident_launch(const char* who, const void* kernel, int threads, int64_t grid, hipStream_t s);
 

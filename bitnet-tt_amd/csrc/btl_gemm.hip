@@ -1220,7 +1220,7 @@ static int decode_waves() {
 // Compute units of the current device (256 on MI355X), cached per device
 // (any thread may fill an entry; every writer stores the same value).  Host
 // code without a GPU (size queries) plans for 256.
-static int device_cus() {
+int device_cus() {
   static std::atomic<int> cached[64];
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) {

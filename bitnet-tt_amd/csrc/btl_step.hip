@@ -186,7 +186,8 @@ struct StepArgs {
   const float* rsin;
   uint16_t* attn_out;
   int64_t off_att;
-  int Hkv, G, S, adjacent;
+  int64_t off_part;  // the attention splits' partials as tagged words, one slot per item
+  int Hkv, G, S, adjacent, smax;
   float scale;
 };
 
@@ -228,6 +229,12 @@ __device__ __forceinline__ uint64_t* out_of(const StepArgs& p, int l, int j) {
 // Tagged words of the attention output (ATT instances): bf16 pairs [32][H / 2].
 __device__ __forceinline__ uint64_t* att_of(const StepArgs& p) {
   return reinterpret_cast<uint64_t*>(p.layers + p.off_att);
+}
+
+// Tagged words of attention item ai's partial (ATT instances): G x 128 fp32
+// outputs, then each head's maximum and sum.
+__device__ __forceinline__ uint64_t* part_of(const StepArgs& p, int ai) {
+  return reinterpret_cast<uint64_t*>(p.layers + p.off_part) + (int64_t)ai * kAtPartFloats;
 }
 
 // Loads of an operand tile.  Every layer reuses the tile's addresses, and a
@@ -994,17 +1001,60 @@ __device__ void step_gemm_op(const StepArgs& p, const StepOp* sops, int l, int g
 // LDS words of the attention instances' GEMM workgroups, above the attention's
 // LDS: the unit index (read back each layer) and a zero (read by the attention).
 constexpr int kStepIdxInt = 20400;
-// Decode attention of user b = ai / Hkv and key-value head hk = ai % Hkv (ATT
-// instances; src/bitnet_tt/inference/generator_batch32.py:728-746), item ai of
-// the layer, run by a GEMM workgroup between its QKV and o_proj units.  The
-// first round of the pair's cached keys and values does not depend on this
-// step, so its loads are issued first; then the new token's rows (the group's G query heads, its
-// key and value head) come in as row b's tagged QKV output words, and the
-// body shared with btl_decode_attention runs on the workgroup (the same code,
-// so the same bits).  Its G x 128 outputs leave as tagged bf16 pairs, which
-// row b's workgroup polls for its o_proj stage, and as the caller's copy.
+// Decode attention item ai of the layer (ATT instances; src/bitnet_tt/
+// inference/generator_batch32.py:728-746): split ai / (M Hkv) of pair
+// ai % (M Hkv), user b and key-value head hk, run by a GEMM workgroup between its QKV
+// and o_proj units.  The first round of the pair's cached keys and values does
+// not depend on this step, so its loads are issued first; then the new token's
+// rows (the group's G query heads, and for split 0 its key and value head)
+// come in as row b's tagged QKV output words, and the body shared with
+// btl_decode_attention runs on the workgroup (the same code, so the same
+// bits).  Its G x 128 outputs leave as tagged bf16 pairs, which row b's
+// workgroup polls for its o_proj stage, and as the caller's copy.  Where the
+// pair's context is split, the other splits hand their partials to split 0 as
+// tagged fp32 words (the data is its own flag), which merges them.  A slot is
+// reused a layer later: its writer has then seen QKV words that depend on this
+// layer's attention output, so split 0 has read it.
+// Split 0's thread (g, d): its output from its own partial and the tagged
+// words of the other splits (items ai + i M Hkv).  Every load of a
+// round is issued before a tag is checked.
+__device__ __forceinline__ uint32_t gather_partials(const StepArgs& p, const AttnSmem& s, int ai, int n,
+                                                    const AttnPartial& mine, uint32_t want, WaitState& ws) {
+  const int tid = threadIdx.x, ml = kAtMaxG * kAtD + 2 * (tid / kAtD);
+  float Ms[kAtMaxSplits], Ls[kAtMaxSplits], Os[kAtMaxSplits];
+#pragma unroll
+  for (int i = 0; i < kAtMaxSplits; ++i) Ms[i] = mine.M, Ls[i] = mine.L, Os[i] = mine.O;
+  const uint64_t* const w0 = part_of(p, ai);
+  unsigned k = 0;
+  while (!ws.dead) {
+    uint64_t o[kAtMaxSplits], m[kAtMaxSplits], l[kAtMaxSplits];
+#pragma unroll
+    for (int i = 1; i < kAtMaxSplits; ++i)
+      if (i < n) {
+        const uint64_t* const w = w0 + (int64_t)i * p.M * p.Hkv * kAtPartFloats;
+        o[i] = ld_coherent(w + tid);
+        m[i] = ld_coherent(w + ml);
+        l[i] = ld_coherent(w + ml + 1);
+      }
+    bool ok = true;
+#pragma unroll
+    for (int i = 1; i < kAtMaxSplits; ++i)
+      if (i < n) {
+        ok = ok && (uint32_t)(o[i] >> 32) == want && (uint32_t)(m[i] >> 32) == want && (uint32_t)(l[i] >> 32) == want;
+        Os[i] = __uint_as_float((uint32_t)o[i]);
+        Ms[i] = __uint_as_float((uint32_t)m[i]);
+        Ls[i] = __uint_as_float((uint32_t)l[i]);
+      }
+    if (__all(ok) || should_stop(p, ++k, ws, WAIT_ATT_WORDS, want)) break;
+    __builtin_amdgcn_s_sleep(BTL_STEP_POLL_SLEEP);
+  }
+  return att_merge(s, tid, n, Ms, Ls, Os);
+}
+
+template <bool SPLIT>
 __device__ void step_attention(const StepArgs& p, int l, int ai, uint32_t E, int32_t* lds, WaitState& ws) {
-  if (ai < 0 || ai >= p.M * p.Hkv) return;
+  const int smax = SPLIT ? p.smax : 1;
+  if (ai < 0 || ai >= p.M * p.Hkv * smax) return;
   const int tid = threadIdx.x;
   AttnSmem& s = *reinterpret_cast<AttnSmem*>(lds);
   AttnPair a;
@@ -1015,18 +1065,23 @@ __device__ void step_attention(const StepArgs& p, int l, int ai, uint32_t E, int
   a.Hkv = p.Hkv;
   a.G = p.G;
   a.S = p.S;
-  a.b = ai / p.Hkv;
-  a.hk = ai % p.Hkv;
-  a.pos = p.pos[a.b];
+  const int pairs = p.M * p.Hkv, pr = SPLIT ? ai % pairs : ai;
+  a.smax = smax;
+  a.split = SPLIT ? ai / pairs : 0;
+  a.b = pr / p.Hkv;
+  a.hk = pr % p.Hkv;
+  a.pos = __builtin_amdgcn_readfirstlane(p.pos[a.b]);
   a.scale = p.scale;
   a.adjacent = p.adjacent;
   // the thread index plus a zero read back from LDS on every call: the body's
   // per-lane values are recomputed in each layer rather than kept (spilled)
   // across the layer loop
   a.tid = tid + *reinterpret_cast<volatile int32_t*>(lds + kStepIdxInt + 1);
+  const int nsplits = SPLIT ? a.splits() : 1;
+  if (a.split != 0 && a.split >= nsplits) return;  // uniform: every thread holds the same position
   if (!a.pos_ok() && tid == 0) set_error_word(p, BAD_POSITION, (uint32_t)(l * 4 + S_O));
   AttnRound r;
-  att_load_round(a, 0, r);
+  att_load_first(a, r);
   STEP_TRACE(l, 0);
   // the new rows: thread t < 6 x 64 takes word t % 64 (two values) of row
   // segment t / 64 (query rows 0..G-1, the key row at kAtMaxG, the value row
@@ -1036,7 +1091,7 @@ __device__ void step_attention(const StepArgs& p, int l, int ai, uint32_t E, int
   const int Hq = p.G * p.Hkv;
   if (tid < (kAtMaxG + 2) * (kAtD / 2)) {
     const int u = tid / (kAtD / 2), w = tid % (kAtD / 2);
-    if (u >= kAtMaxG || u < p.G) {
+    if (u >= kAtMaxG ? a.split == 0 : u < p.G) {
       const int head = u < kAtMaxG ? a.hk * p.G + u : u == kAtMaxG ? Hq + a.hk : Hq + p.Hkv + a.hk;
       const uint64_t* wp = row + head * (kAtD / 2) + w;
       unsigned n = 0;
@@ -1052,7 +1107,26 @@ __device__ void step_attention(const StepArgs& p, int l, int ai, uint32_t E, int
   }
   lds_barrier();  // the new rows are in LDS (the cache loads stay in flight)
   STEP_TRACE(l, 1);
-  const uint32_t o = att_body(a, s, r, l == BTL_STEP_TRACE_LAYER);
+  AttnPartial part;
+  uint32_t o = att_body(a, s, r, part, l == BTL_STEP_TRACE_LAYER);
+  if (SPLIT && nsplits > 1) {
+    const uint32_t ptag = step_tag(E, l, 0);
+    const int g = tid / kAtD;
+    if (a.split != 0) {
+      if (g < p.G) {
+        uint64_t* const w = part_of(p, ai);
+        const uint64_t t = (uint64_t)ptag << 32;
+        st_coherent(w + tid, t | __float_as_uint(part.O));
+        if (tid % kAtD == 0) {
+          st_coherent(w + kAtMaxG * kAtD + 2 * g, t | __float_as_uint(part.M));
+          st_coherent(w + kAtMaxG * kAtD + 2 * g + 1, t | __float_as_uint(part.L));
+        }
+      }
+      lds_barrier();  // the LDS is the next BitLinear's again
+      return;
+    }
+    if (g < p.G) o = gather_partials(p, s, ai, nsplits, part, ptag, ws);
+  }
   const uint32_t pair = o | (xor_partner_u<1>(o) << 16);  // dims d, d + 1 of a head (a DPP lane swap)
   if (tid < p.G * kAtD && (tid & 1) == 0) {
     const int col = a.hk * p.G * kAtD + tid;  // heads hk G + tid / 128, dimension tid % 128
@@ -1064,22 +1138,25 @@ __device__ void step_attention(const StepArgs& p, int l, int ai, uint32_t E, int
 }
 
 
-// The first GEMM unit with an attention item: the items take the last M * Hkv
-// units, which at the 2B shape (160 items, 60 QKV units of 224) have no QKV
+// The first GEMM unit with an attention item: the items (smax per user and
+// key-value head) take the last units, which at the 2B shape (160 items, 60 QKV units of 224) have no QKV
 // work, so each issues its cached keys and values at the start of the layer.
 __device__ __forceinline__ int step_first_att(const StepArgs& p) {
-  return (int)gridDim.x - kStepRows - p.M * p.Hkv;
+  return (int)gridDim.x - kStepRows - p.M * p.Hkv * p.smax;
 }
 
-// NQ: superblocks per wave of a unit of QKV, O and GU (K = H); NDN: of DN (K = F).
-template <int NQ, int NDN, bool ATT>
+// NQ: superblocks per wave of a unit of QKV, O and GU (K = H); NDN: of DN
+// (K = F).  ATT: 0 without the decode attention, 1 with it, 2 with it and the
+// pairs' contexts split over several units (an instance of its own: one with
+// both, at 253 registers without the split, would spill in every step).
+template <int NQ, int NDN, int ATT>
 __device__ void step_gemm(const StepArgs& p, const StepOp* sops, int gi, uint32_t E, int32_t* lds) {
   // Word kStError + 64 of the workspace: bit 0 makes every GEMM unit take the
   // re-read path of its sentinel check (a test of that rare path; the results
   // are the same bits).
   WaitState ws{false, (__builtin_amdgcn_readfirstlane(p.error[16]) & 1u) != 0u};
   v4i wa[kStepWSlots], wb[kStepWSlots];
-  load_unit_weights<S_QKV, NQ, ATT>(p, sops, 0, gi, wa);
+  load_unit_weights<S_QKV, NQ, ATT != 0>(p, sops, 0, gi, wa);
   if (threadIdx.x == 0) {
     lds[kStepIdxInt] = gi;
     lds[kStepIdxInt + 1] = 0;  // the attention body's opaque zero
@@ -1097,18 +1174,18 @@ __device__ void step_gemm(const StepArgs& p, const StepOp* sops, int gi, uint32_
     // arrive microseconds later, through the rows' o_proj stage.
     const int ai = ATT ? gi - step_first_att(p) : -1;
     const bool att_unit = ai >= 0;
-    step_gemm_op<S_QKV, NQ, S_O, NQ, ATT>(p, sops, l, gi, E, wa, wb, att_unit ? p.L : l, lds, ws);
+    step_gemm_op<S_QKV, NQ, S_O, NQ, ATT != 0>(p, sops, l, gi, E, wa, wb, att_unit ? p.L : l, lds, ws);
     if (att_unit) {
-      step_attention(p, l, ai, E, lds, ws);
-      load_unit_weights<S_O, NQ, ATT>(p, sops, l, gi, wb);
+      step_attention<ATT == 2>(p, l, ai, E, lds, ws);
+      load_unit_weights<S_O, NQ, ATT != 0>(p, sops, l, gi, wb);
     }
-    step_gemm_op<S_O, NQ, S_GU, NQ, ATT>(p, sops, l, gi, E, wb, wa, l, lds, ws);
-    step_gemm_op<S_GU, NQ, S_DN, NDN, ATT>(p, sops, l, gi, E, wa, wb, l, lds, ws);
-    step_gemm_op<S_DN, NDN, S_QKV, NQ, ATT>(p, sops, l, gi, E, wb, wa, l + 1, lds, ws);
+    step_gemm_op<S_O, NQ, S_GU, NQ, ATT != 0>(p, sops, l, gi, E, wb, wa, l, lds, ws);
+    step_gemm_op<S_GU, NQ, S_DN, NDN, ATT != 0>(p, sops, l, gi, E, wa, wb, l, lds, ws);
+    step_gemm_op<S_DN, NDN, S_QKV, NQ, ATT != 0>(p, sops, l, gi, E, wb, wa, l + 1, lds, ws);
   }
 }
 
-template <int CF, int NQ, int NDN, bool ATT>
+template <int CF, int NQ, int NDN, int ATT>
 __global__ __launch_bounds__(512) void k_decode_step(StepArgs p) {
   // GEMM: reductions [8][2][16][64] int32 and 32 a/127; rows: 16 words.  The op table
   // (up to 16 KiB) is copied into LDS above them, so reading a weight address or a
@@ -1134,7 +1211,7 @@ __global__ __launch_bounds__(512) void k_decode_step(StepArgs p) {
   const uint32_t E = p.epoch[b] + 1u;  // this launch (written by the previous launch of the step)
   if (b < kStepRows) {
     float* f = reinterpret_cast<float*>(lds);
-    step_row<CF, ATT>(p, sops, b, E, f, f + kActWaves);
+    step_row<CF, ATT != 0>(p, sops, b, E, f, f + kActWaves);
   } else {
     step_gemm<NQ, NDN, ATT>(p, sops, b - kStepRows, E, lds);
   }
@@ -1222,7 +1299,7 @@ __global__ __launch_bounds__(512) void k_decode_step_floor(StepArgs p) {
 
 // ---------------------------------------------------------------- host ----
 struct StepSizes {
-  int64_t off_xa[kStepOps], tiles_end, off_flag, off_out[kStepOps], off_att, layer_bytes, total;
+  int64_t off_xa[kStepOps], tiles_end, off_flag, off_out[kStepOps], off_att, off_part, layer_bytes, total;
 };
 
 static StepSizes step_sizes(int64_t H, int64_t F, int64_t NQKV) {
@@ -1244,6 +1321,8 @@ static StepSizes step_sizes(int64_t H, int64_t F, int64_t NQKV) {
   }
   z.off_att = off;  // the attention output's tagged words (ATT instances)
   off += round_up(32 * (H / 2) * 8, 4096);
+  z.off_part = off;  // the attention splits' partials
+  off += (int64_t)kAtSplitItems * kAtPartFloats * 8;
   z.layer_bytes = round_up(off, 65536);
   z.total = kStHeader + z.layer_bytes;
   return z;
@@ -1257,14 +1336,14 @@ static int step_grid() {
 }
 
 // The step's instance for F (the down projection's row chunks per thread),
-// with or without the decode attention.
-static void (*step_kernel_fn(int64_t F, bool att))(StepArgs) {
+// without the decode attention (0), with it (1) or with it split (2).
+static void (*step_kernel_fn(int64_t F, int att))(StepArgs) {
   const int cf = act_cpt(F);
-  if (cf == 1) return att ? k_decode_step<1, 3, 7, true> : k_decode_step<1, 3, 7, false>;
-  if (cf == 2) return att ? k_decode_step<2, 3, 7, true> : k_decode_step<2, 3, 7, false>;
+  if (cf == 1) return att == 2 ? k_decode_step<1, 3, 7, 2> : att ? k_decode_step<1, 3, 7, 1> : k_decode_step<1, 3, 7, 0>;
+  if (cf == 2) return att == 2 ? k_decode_step<2, 3, 7, 2> : att ? k_decode_step<2, 3, 7, 1> : k_decode_step<2, 3, 7, 0>;
   return nullptr;
 }
-static const void* step_kernel(int64_t F, bool floor, bool att = false) {
+static const void* step_kernel(int64_t F, bool floor, int att = 0) {
   const int cf = act_cpt(F);
   if (floor) return cf == 1 ? reinterpret_cast<const void*>(k_decode_step_floor<1>)
                             : reinterpret_cast<const void*>(k_decode_step_floor<2>);
@@ -1321,7 +1400,7 @@ static StepArgs step_args(int64_t M, int64_t H, int64_t F, int64_t NQKV, int64_t
   return a;
 }
 
-static int launch_step(const StepArgs& a, int64_t F, bool att, const char* who, hipStream_t s) {
+static int launch_step(const StepArgs& a, int64_t F, int att, const char* who, hipStream_t s) {
   void (*k)(StepArgs) = step_kernel_fn(F, att);
   if (!k) return set_error(BTL_ERR_SHAPE, "%s: no kernel instance for F=%lld", who, (long long)F);
   const int grid = step_grid();
@@ -1434,7 +1513,7 @@ int btl_decode_step(int64_t M, int64_t H, int64_t F, int64_t NQKV, int64_t L, fl
                      (long long)z.total);
   StepArgs a = step_args(M, H, F, NQKV, L, eps, hidden, qkv_out, ffn_h, (char*)workspace, z);
   a.attn = attn;
-  return launch_step(a, F, false, "btl_decode_step", (hipStream_t)stream);
+  return launch_step(a, F, 0, "btl_decode_step", (hipStream_t)stream);
 }
 
 int btl_decode_step_attention_prepare(int64_t M, int64_t H, int64_t F, int64_t NQKV, int64_t L,
@@ -1502,12 +1581,14 @@ int btl_decode_step_full(int64_t M, int64_t H, int64_t F, int64_t NQKV, int64_t 
   a.rsin = rope_sin;
   a.attn_out = attn_out;
   a.off_att = z.off_att;
+  a.off_part = z.off_part;
+  a.smax = att_max_splits(M * Hkv, S, step_grid());
   a.Hkv = (int)Hkv;
   a.G = (int)(Hq / Hkv);
   a.S = (int)S;
   a.adjacent = rope_adjacent ? 1 : 0;
   a.scale = scale;
-  return launch_step(a, F, true, "btl_decode_step_full", (hipStream_t)stream);
+  return launch_step(a, F, a.smax > 1 ? 2 : 1, "btl_decode_step_full", (hipStream_t)stream);
 }
 
 int btl_decode_step_floor(int64_t M, int64_t H, int64_t F, int64_t NQKV, int64_t L, void* workspace,

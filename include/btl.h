@@ -373,7 +373,10 @@ int btl_lm_head(const uint16_t* xn, int64_t M, int64_t K, int64_t V, const uint1
  * D = 128, H / Hkv <= 4.  The workspace holds one int32 at
  * btl_decode_attention_error_offset (zero-filled before the first call): it
  * becomes non-zero when a position is outside [0, S) (that user's output is
- * then zero and its caches are not written). */
+ * then zero and its caches are not written).  Where B * Hkv pairs leave CUs
+ * idle and S > 512, contexts are split over several workgroups, whose arrival
+ * counters (zero between calls) and partials lie behind it: zero-fill the
+ * whole workspace, and order the calls that share one. */
 int64_t btl_decode_attention_workspace_bytes(int64_t B, int64_t H, int64_t Hkv, int64_t S);
 int64_t btl_decode_attention_error_offset(int64_t B, int64_t Hkv);
 int btl_decode_attention(const uint16_t* qkv, int64_t B, int64_t H, int64_t Hkv, int64_t D, int64_t S,

@@ -345,3 +345,53 @@ def test_persistent_full_step_matches_step_full_2b(orc):
     finally:
         ws[off:off + 4] = 0
         torch.cuda.synchronize()
+
+
+# (users, query heads, kv heads, cache length, positions): the edges of one
+# round (511..513 cached positions), of the blocks of 64 and of the splits'
+# ranges; 8, 5, 2 and 1 splits per pair; an out-of-range user among split ones
+# is left to test_position_out_of_range_is_flagged's single-split shape.
+SPLIT_SHAPES = [
+    (1, 4, 1, 4096, [4095]),
+    (4, 20, 5, 4096, [0, 511, 512, 4095]),
+    (6, 6, 3, 2048, [513, 575, 576, 577, 1023, 1024]),
+    (3, 8, 8, 1000, [999, 640, 513]),
+    (16, 20, 5, 1024, [1023 - 37 * i for i in range(16)]),
+    (23, 20, 5, 640, [639 - i for i in range(23)]),
+]
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,S,pos", SPLIT_SHAPES)
+def test_split_contexts(orc, B, Hq, Hkv, S, pos):
+    """Contexts split over several workgroups against the oracle, twice on the
+    same workspace (the arrival counters are left clean)."""
+    print(f"split attention B={B} Hq={Hq} Hkv={Hkv} S={S}", flush=True)
+    for seed in (51, 52):
+        att, cache, got, ref, kc, vc, kc2, vc2 = run(orc, B, Hq, Hkv, S, pos, seed == 52, seed)
+        att.check()
+        check(orc, got, ref, cache, kc2, vc2)
+
+
+@pytest.mark.parametrize("batch,kv,S", [(1, 1, 4096), (5, 2, 1024), (26, 1, 640)])
+def test_persistent_full_step_split_contexts(orc, batch, kv, S):
+    """The one-launch step with split contexts against step_full, bit for bit,
+    three steps in a row at moving positions (the partials' words are reused by
+    every layer and launch)."""
+    from bitnet_tt.config import BitNetMiniConfig
+    from bitnet_tt.decode import BitLinearDecodeStep
+
+    cfg = BitNetMiniConfig(num_layers=2, num_attention_heads=4, num_key_value_heads=kv, hidden_size=512,
+                           intermediate_size=512)
+    print(f"persistent full step, split contexts: batch {batch} kv {kv} S {S}", flush=True)
+    step = BitLinearDecodeStep.random_init(cfg, H.dev(), seed=93, batch=batch).alloc_buffers(seed=94)
+    step.alloc_attention(max_seq_len=S)
+    for back in (1, S // 2 - 60, 2):
+        step.pos.copy_(torch.tensor([max(0, S - back - 13 * i) for i in range(batch)], dtype=torch.int32))
+        state = _full_state(step)
+        step.step_full()
+        step.check()
+        ref = _outputs(step)
+        _restore(step, state)
+        step.step_persistent_full()
+        step.check()
+        _compare(_outputs(step), ref, f"split contexts, back {back}")
