@@ -86,6 +86,7 @@ EXPORTS = {
     "btl_fused_error_offset": ([], _I64),
     "btl_weight_quant_scratch_bytes": ([_I64], _I64),
     "btl_weight_quant_ternary": ([_P, _I64, _F, _P, _P, _P, _SZ, _P], _I),
+    "btl_weight_quant_pack": ([_P, _I64, _I64, _F, _P, _P, _P, _SZ, _P], _I),
     "btl_pack_tiles": ([_P, _I64, _I64, _P, _P], _I),
     "btl_unpack_tiles": ([_P, _I64, _I64, _P, _P], _I),
     "btl_repack": ([_P, _I64, _I64, _P, _P], _I),

@@ -188,3 +188,31 @@ def repack_for_gemm(packed, in_features: int, out_features: int):
         "btl_repack",
     )
     return wdev
+
+
+def quantize_for_gemm(weight, eps: float = 1e-5):
+    """Latent weight (out, in), a float32 ROCm tensor -> (the GEMM's device
+    layout, absmean scale as a float): ``weight_quant_ternary``, the tile format
+    and :func:`repack_for_gemm` in one pass over the weight, the same bits.
+    Synchronises (the scale comes back)."""
+    import torch
+
+    from .. import _native as N
+
+    N.require_cuda(weight, "weight")
+    if weight.dtype != torch.float32 or weight.dim() != 2:
+        raise ValueError("weight must be a 2-D float32 tensor (out_features, in_features)")
+    out_f, in_f = weight.shape
+    if in_f % 32 or out_f % 32:
+        raise ValueError("K/N must be multiples of 32")  # bitlinear.py:226, 276
+    dev = weight.device
+    L = N.lib()
+    wdev = torch.empty((out_f // 32, (in_f + 127) // 128, 256), dtype=torch.int32, device=dev)
+    nb = int(L.btl_weight_quant_scratch_bytes(weight.numel())) // 4
+    scratch = torch.empty(nb + 1, dtype=torch.float32, device=dev)  # block sums, then the scale
+    N.check(
+        L.btl_weight_quant_pack(N.ptr(weight), out_f, in_f, eps, N.ptr(wdev), scratch.data_ptr() + 4 * nb,
+                                N.ptr(scratch), 4 * nb, N.stream_of(dev)),
+        "btl_weight_quant_pack",
+    )
+    return wdev, float(scratch[nb].item())

@@ -14,7 +14,7 @@ from __future__ import annotations
 
 import numpy as np
 
-from ..kernels.pack import pack_ternary_tilized_device, repack_for_gemm
+from ..kernels.pack import pack_ternary_tilized_device, quantize_for_gemm, repack_for_gemm
 from ..ternary_matmul import PackedTernaryWeight, ternary_matmul, ternary_matmul_into
 from ..utils.quantization import weight_quant_ternary
 
@@ -104,7 +104,13 @@ class Linear:
 
         dev = _device(self.device)
         if isinstance(weight, torch.Tensor) and weight.is_cuda:
-            q, scale = weight_quant_ternary(weight.to(torch.float32).contiguous())
+            w = weight.to(torch.float32).contiguous()
+            if dev == w.device and w.dim() == 2 and w.data_ptr() % 16 == 0:
+                self._check_shape(*w.shape)
+                data, self.weight_scale = quantize_for_gemm(w)
+                self.weight = PackedTernaryWeight(data, self.in_features, self.out_features, (self.weight_scale,))
+                return
+            q, scale = weight_quant_ternary(w)
         else:
             q, scale = weight_quant_ternary(np.asarray(weight).astype(np.float32))
         self._check_shape(*q.shape)

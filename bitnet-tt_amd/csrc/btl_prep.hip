@@ -105,7 +105,7 @@ int check_coresident_launch(const char* who, const void* kernel, int threads, in
 // block is summed pairwise: blocks of < 8 sequentially, blocks of <= 128 with
 // eight strided accumulators combined as ((r0+r1)+(r2+r3))+((r4+r5)+(r6+r7))
 // plus a sequential tail, larger blocks split at n/2 rounded down to a
-// multiple of 8.  One thread reproduces that tree for one 8192-block.
+// multiple of 8.
 __device__ float pw_leaf_abs(const float* a, int n) {
   if (n < 8) {
     float r = 0.0f;
@@ -116,6 +116,7 @@ __device__ float pw_leaf_abs(const float* a, int n) {
 #pragma unroll
   for (int j = 0; j < 8; ++j) r[j] = fabsf(a[j]);
   int i = 8;
+#pragma unroll 4
   for (; i < n - (n % 8); i += 8) {
 #pragma unroll
     for (int j = 0; j < 8; ++j) r[j] += fabsf(a[i + j]);
@@ -125,58 +126,63 @@ __device__ float pw_leaf_abs(const float* a, int n) {
   return res;
 }
 
-__device__ float pw_abs(const float* a, int n) {
-  // Post-order walk of the split tree with an explicit stack (depth <= 8
-  // for n <= 8192).
-  int off[12], len[12], stage[12];
-  float left[12];
-  int sp = 0;
-  off[0] = 0;
-  len[0] = n;
-  stage[0] = 0;
-  float res = 0.0f;
-  bool have = false;
-  for (;;) {
-    if (!have) {
-      const int o = off[sp], l = len[sp];
-      if (l <= 128) {
-        res = pw_leaf_abs(a + o, l);
-        have = true;
-        if (--sp < 0) return res;
-        continue;
-      }
-      int n2 = l / 2;
-      n2 -= n2 % 8;
-      stage[sp] = 1;
-      ++sp;
-      off[sp] = o;
-      len[sp] = n2;
-      stage[sp] = 0;
-    } else if (stage[sp] == 1) {
-      left[sp] = res;
-      stage[sp] = 2;
-      const int o = off[sp], l = len[sp];
-      int n2 = l / 2;
-      n2 -= n2 % 8;
-      ++sp;
-      off[sp] = o + n2;
-      len[sp] = l - n2;
-      stage[sp] = 0;
-      have = false;
-    } else {
-      res = left[sp] + res;
-      if (--sp < 0) return res;
-    }
-  }
+// One step of the wave's walk back up the split tree: lanes `D` apart hold
+// the two subtrees of a node; a side that is absent (its parent was a leaf)
+// adds nothing.
+template <int D>
+__device__ __forceinline__ void pw_join(float& v, uint32_t& has) {
+  const float o = xor_partner<D>(v);
+  const uint32_t oh = xor_partner_u<D>(has);
+  v = has ? (oh ? v + o : v) : o;
+  has |= oh;
 }
 
-// Blocks b0, b0 + 1, ... one thread each (the partial last block).
-__global__ void k_wq_block_sums(const float* __restrict__ w, int64_t n, float* __restrict__ part, int64_t b0) {
-  const int64_t b = b0 + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+// Blocks b0, b0 + 1, ... of any length and alignment (the partial last block;
+// every block of an unaligned array), one wave each.  A block of 8192 splits
+// at most seven times before its parts are <= 128 long: lane j takes the node
+// that the bits of j (first split first) lead to, or, where a leaf comes
+// earlier, the lane whose remaining bits are 0 takes that; nodes still over
+// 128 long are two leaves.  Six joins (float addition is commutative, so
+// which lane of a pair holds the left part does not matter) then give the
+// same sum as the sequential walk.  (One thread walking the tree took 60-80 us
+// for a last block, of any weight whose size is no multiple of 8192.)
+__global__ __launch_bounds__(256) void k_wq_block_sums(const float* __restrict__ w, int64_t n,
+                                                       float* __restrict__ part, int64_t b0) {
+  const int64_t b = b0 + (((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+  const int lane = threadIdx.x & 63;
   const int64_t start = b * 8192;
-  if (start >= n) return;
-  const int len = (int)((n - start) < 8192 ? (n - start) : 8192);
-  part[b] = pw_abs(w + start, len);
+  if (start >= n) return;  // wave-uniform
+  int o = 0, l = (int)((n - start) < 8192 ? (n - start) : 8192);
+  uint32_t has = 1u;
+  for (int d = 5; d >= 0; --d) {
+    const bool right = (lane >> d) & 1;
+    if (l <= 128) {
+      if (right) has = 0u;
+    } else {
+      int n2 = l / 2;
+      n2 -= n2 % 8;
+      o += right ? n2 : 0;
+      l = right ? l - n2 : n2;
+    }
+  }
+  const float* a = w + start + o;
+  float v = 0.0f;
+  if (has) {
+    if (l <= 128) {
+      v = pw_leaf_abs(a, l);
+    } else {
+      int n2 = l / 2;
+      n2 -= n2 % 8;
+      v = pw_leaf_abs(a, n2) + pw_leaf_abs(a + n2, l - n2);
+    }
+  }
+  pw_join<1>(v, has);
+  pw_join<2>(v, has);
+  pw_join<4>(v, has);
+  pw_join<8>(v, has);
+  pw_join<16>(v, has);
+  pw_join<32>(v, has);
+  if (lane == 0) part[b] = v;
 }
 
 // Full 8192-blocks, one wave each.  The split tree of 8192 is balanced (every
@@ -184,7 +190,7 @@ __global__ void k_wq_block_sums(const float* __restrict__ w, int64_t n, float* _
 // (elements 128 j .. 128 j + 127) as pw_leaf_abs does, and each of the six
 // levels above adds adjacent subtrees, one xor butterfly step (float addition
 // is commutative, so which lane of a pair holds the left subtree does not
-// matter).  The same sums as the one-thread walk, in a 64th of the passes.
+// matter).
 __global__ __launch_bounds__(256) void k_wq_block_sums_wave(const float* __restrict__ w, int64_t nfull,
                                                             float* __restrict__ part) {
   const int64_t b = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
@@ -215,7 +221,8 @@ __global__ __launch_bounds__(256) void k_wq_block_sums_wave(const float* __restr
 
 // The blocks' sums in block order (numpy adds its buffered blocks one after
 // another): 256 threads stage up to 8192 partials at a time in LDS, and
-// thread 0 adds them in order, four per LDS read.
+// thread 0 adds them in order, four per LDS read.  The chain of dependent
+// adds sets the time, 4 ns each (reading ahead changes nothing).
 __global__ __launch_bounds__(256) void k_wq_finalize(const float* __restrict__ part, int64_t nblocks, int64_t n,
                                                      float eps, float* __restrict__ scale_out) {
   __shared__ __attribute__((aligned(16))) float sp[8192];
@@ -246,13 +253,72 @@ __global__ __launch_bounds__(256) void k_wq_finalize(const float* __restrict__ p
   scale_out[0] = mean > eps ? mean : eps;
 }
 
+// q = clip(rne(w / s), -1, 1).  The correctly rounded w / s exceeds 0.5 exactly
+// where w > 0.5 s (0.5 s is exact, and the next float above it already rounds
+// above 0.5), so two compares replace the division; a NaN is -1, as fmaxf
+// takes it.  Scales whose half is not exact, or infinite ones, divide.
+__device__ __forceinline__ bool tern_by_compare(float s) { return s >= 1e-30f && s <= 3e38f; }
+__device__ __forceinline__ int tern_of(float w, float t) { return (w > t ? 1 : 0) - (w >= -t ? 0 : 1); }
+__device__ __forceinline__ int tern_by_division(float w, float s) {
+  return (int)fminf(fmaxf(rintf(w / s), -1.0f), 1.0f);  // correctly rounded division (HIP default)
+}
+
 __global__ void k_wq_quant(const float* __restrict__ w, int64_t n, const float* __restrict__ scale,
                            int8_t* __restrict__ q) {
   const float s = scale[0];
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-    float r = rintf(w[i] / s);  // correctly rounded division (HIP default)
-    r = fminf(fmaxf(r, -1.0f), 1.0f);
-    q[i] = (int8_t)(int)r;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
+    q[i] = (int8_t)tern_by_division(w[i], s);
+}
+
+// The latent weight [N][K] quantised and written in the GEMM's device layout
+// (below) in one pass: the codes never go through memory as bytes or tiles.
+// One wave per column tile and superblock: 32 columns x 128 k, two columns of
+// 512 contiguous bytes per load instruction, all 16 loads in flight.  Lane l
+// holds k 4 (l & 31) .. + 3 of column 2 i + (l >> 5) in load i: four codes of
+// the word of k-chunk (l & 31) / 4, which four lanes make up together; of
+// every four loads each of them keeps one, and writes it.
+// Measured on MI355X, 2560 x 6912: 14.5 us (5.2 TB/s) where quantising to bytes
+// (28.9 us), packing the tiles (14.0) and repacking them (14.0) took 57.  (Adding
+// the block sums here too, under the first loads, gave 25.6 us against 26.8 with
+// the launch before it: not worth a second form of the kernel.)
+__global__ __launch_bounds__(256) void k_wq_pack(const float* __restrict__ w, int64_t K, int64_t KS, int64_t nsb,
+                                                 const float* __restrict__ scale, uint32_t* __restrict__ wdev) {
+  const int64_t sbi = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;  // nt * KS + ks
+  const int lane = threadIdx.x & 63;
+  if (sbi >= nsb) return;  // wave-uniform
+  const int64_t nt = sbi / KS, ks = sbi % KS;
+  const int64_t k = ks * 128 + (lane & 31) * 4;
+  const bool in = k < K;
+  const float* src = w + (nt * 32 + (lane >> 5)) * K + k;
+  float4 v[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i)
+    v[i] = in ? *reinterpret_cast<const float4*>(src + 2 * i * K) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  const float s = scale[0];
+  const int sh = 2 * (lane & 3);  // code j = 4 (l & 3) + c of a word lies at bit 8 c + 2 (j >> 2)
+  uint32_t mine[4];
+  auto pack = [&](auto code) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      uint32_t d = (uint32_t)(code(v[i].x) + 1) | ((uint32_t)(code(v[i].y) + 1) << 8) |
+                   ((uint32_t)(code(v[i].z) + 1) << 16) | ((uint32_t)(code(v[i].w) + 1) << 24);
+      if (!in) d = 0x01010101u;  // weight 0 past K
+      d <<= sh;
+      d |= xor_partner_u<1>(d);
+      d |= xor_partner_u<2>(d);
+      if ((i & 3) == 0 || (lane & 3) == (i & 3)) mine[i >> 2] = d;
+    }
+  };
+  const float t = 0.5f * s;
+  if (tern_by_compare(s))
+    pack([&](float x) { return tern_of(x, t); });
+  else
+    pack([&](float x) { return tern_by_division(x, s); });
+  const int kk = (lane & 31) >> 2;
+#pragma unroll
+  for (int a = 0; a < 4; ++a) {
+    const int col = 2 * (4 * a + (lane & 3)) + (lane >> 5);
+    wdev[((sbi * 64) + (kk & 1) * 32 + col) * 4 + (kk >> 1)] = mine[a];
   }
 }
 
@@ -369,30 +435,55 @@ int64_t btl_weight_quant_scratch_bytes(int64_t n) {
   return ((n + 8191) / 8192) * (int64_t)sizeof(float);
 }
 
+static int check_weight_quant(const char* who, const float* w, int64_t n, const float* scale_out, const void* scratch,
+                              size_t scratch_bytes) {
+  if (n <= 0) return set_error(BTL_ERR_SHAPE, "%s: n=%lld", who, (long long)n);
+  if (!aligned(scratch, 4) || !aligned(scale_out, 4) || !aligned(w, 4))
+    return set_error(BTL_ERR_ALIGN, "%s: float buffers must be 4-byte aligned", who);
+  if ((int64_t)scratch_bytes < btl_weight_quant_scratch_bytes(n))
+    return set_error(BTL_ERR_WORKSPACE, "%s: scratch %zu < %lld", who, scratch_bytes,
+                     (long long)btl_weight_quant_scratch_bytes(n));
+  return BTL_OK;
+}
+// The absmean scale of w[0 .. n) in numpy's summation order.
+static void launch_scale(const float* w, int64_t n, float eps, float* scale_out, float* part, hipStream_t s) {
+  const int64_t nb = (n + 8191) / 8192, nfull = aligned(w, 16) ? n / 8192 : 0;
+  // full blocks by float4 loads (w 16-byte aligned), the others element by element
+  if (nfull > 0) hipLaunchKernelGGL(k_wq_block_sums_wave, dim3(grid_for(nfull * 64, 256)), dim3(256), 0, s, w, nfull, part);
+  if (nb > nfull)
+    hipLaunchKernelGGL(k_wq_block_sums, dim3(grid_for((nb - nfull) * 64, 256)), dim3(256), 0, s, w, n, part, nfull);
+  hipLaunchKernelGGL(k_wq_finalize, dim3(1), dim3(256), 0, s, part, nb, n, eps, scale_out);
+}
+
 int btl_weight_quant_ternary(const float* w, int64_t n, float eps, int8_t* q, float* scale_out, void* scratch,
                              size_t scratch_bytes, btl_stream_t stream) {
   clear_error();
   if (!w || !q || !scale_out || !scratch) return set_error(BTL_ERR_NULL, "btl_weight_quant_ternary: null pointer");
-  if (n <= 0) return set_error(BTL_ERR_SHAPE, "btl_weight_quant_ternary: n=%lld", (long long)n);
-  if (!aligned(scratch, 4) || !aligned(scale_out, 4) || !aligned(w, 4))
-    return set_error(BTL_ERR_ALIGN, "btl_weight_quant_ternary: float buffers must be 4-byte aligned");
-  if ((int64_t)scratch_bytes < btl_weight_quant_scratch_bytes(n))
-    return set_error(BTL_ERR_WORKSPACE, "btl_weight_quant_ternary: scratch %zu < %lld", scratch_bytes,
-                     (long long)btl_weight_quant_scratch_bytes(n));
+  const int rc = check_weight_quant("btl_weight_quant_ternary", w, n, scale_out, scratch, scratch_bytes);
+  if (rc) return rc;
   hipStream_t s = (hipStream_t)stream;
-  const int64_t nb = (n + 8191) / 8192, nfull = n / 8192;
-  float* part = (float*)scratch;
-  // full blocks one wave each (float4 loads: w 16-byte aligned), else one thread a block
-  if (aligned(w, 16)) {
-    if (nfull > 0) hipLaunchKernelGGL(k_wq_block_sums_wave, dim3(grid_for(nfull * 64, 256)), dim3(256), 0, s, w, nfull, part);
-    if (nb > nfull) hipLaunchKernelGGL(k_wq_block_sums, dim3(1), dim3(64), 0, s, w, n, part, nfull);
-  } else {
-    hipLaunchKernelGGL(k_wq_block_sums, dim3(grid_for(nb, 64)), dim3(64), 0, s, w, n, part, (int64_t)0);
-  }
-  hipLaunchKernelGGL(k_wq_finalize, dim3(1), dim3(256), 0, s, part, nb, n, eps, scale_out);
+  launch_scale(w, n, eps, scale_out, (float*)scratch, s);
   const int64_t blocks = grid_for(n, 256) < 65536 ? grid_for(n, 256) : 65536;
   hipLaunchKernelGGL(k_wq_quant, dim3((unsigned)blocks), dim3(256), 0, s, w, n, scale_out, q);
   return check_launch("btl_weight_quant_ternary");
+}
+
+int btl_weight_quant_pack(const float* w, int64_t N, int64_t K, float eps, uint32_t* wdev, float* scale_out,
+                          void* scratch, size_t scratch_bytes, btl_stream_t stream) {
+  clear_error();
+  if (!w || !wdev || !scale_out || !scratch) return set_error(BTL_ERR_NULL, "btl_weight_quant_pack: null pointer");
+  if (K <= 0 || N <= 0 || K % 32 || N % 32 || K > BTL_MAX_K || N > (1 << 24))
+    return set_error(BTL_ERR_SHAPE, "btl_weight_quant_pack: K=%lld (<= %d) and N=%lld must be positive multiples of 32",
+                     (long long)K, BTL_MAX_K, (long long)N);
+  const int rc = check_weight_quant("btl_weight_quant_pack", w, N * K, scale_out, scratch, scratch_bytes);
+  if (rc) return rc;
+  if (!aligned(w, 16) || !aligned(wdev, 16))
+    return set_error(BTL_ERR_ALIGN, "btl_weight_quant_pack: w and wdev must be 16-byte aligned");
+  hipStream_t s = (hipStream_t)stream;
+  launch_scale(w, N * K, eps, scale_out, (float*)scratch, s);
+  const int64_t nsb = N / 32 * ksb(K);
+  hipLaunchKernelGGL(k_wq_pack, dim3(grid_for(nsb * 64, 256)), dim3(256), 0, s, w, K, ksb(K), nsb, scale_out, wdev);
+  return check_launch("btl_weight_quant_pack");
 }
 
 int btl_pack_tiles(const int8_t* w, int64_t out_f, int64_t in_f, uint8_t* packed, btl_stream_t stream) {

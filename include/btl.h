@@ -113,6 +113,14 @@ int64_t btl_weight_quant_scratch_bytes(int64_t n);
 int btl_weight_quant_ternary(const float* w, int64_t n, float eps, int8_t* q, float* scale_out,
                              void* scratch, size_t scratch_bytes, btl_stream_t stream);
 
+/* btl_weight_quant_ternary of a latent weight [N][K] (out x in) with the codes
+ * written straight into the device layout that btl_pack_tiles and btl_repack
+ * would make of them (btl_devlayout_words(K, N) words, bit-identical).  N and K
+ * multiples of 32, w and wdev 16-byte aligned; the scratch is that of
+ * btl_weight_quant_ternary for N * K elements. */
+int btl_weight_quant_pack(const float* w, int64_t N, int64_t K, float eps, uint32_t* wdev, float* scale_out,
+                          void* scratch, size_t scratch_bytes, btl_stream_t stream);
+
 /* pack_ternary_tilized (src/bitnet_tt/kernels/pack.py:101-155): quantised
  * (out_features, in_features) int8 -> 2-bit tiles of the transposed matrix,
  * tile t = kt*Nt + nt, faces f0..f3, codes {0:00,+1:01,-1:10}, MSB first,

@@ -353,3 +353,32 @@ def test_lm_head_sizes_and_argument_checks(L):
     assert call(nbytes=100) == WS
     assert L.btl_lm_head_repack(None, 100, 256, FAKE, None) == NULL
     assert L.btl_lm_head_repack(FAKE, 100, 250, FAKE, None) == SHAPE
+
+
+def test_weight_quant_pack_argument_checks(L):
+    """The one-pass load refuses what the three passes refuse: NULL (1), shapes
+    that are no multiples of 32 or too large (2), misalignment (3), a short
+    scratch (4)."""
+    def call(w=FAKE, n=64, k=96, out=FAKE, scratch=8):
+        return L.btl_weight_quant_pack(_p(w), n, k, 1e-5, _p(out), _p(FAKE), _p(FAKE), scratch, None)
+
+    assert call(w=0) == 1 and call(out=0) == 1
+    assert call(n=33) == 2 and call(k=100) == 2 and call(k=16416) == 2 and call(n=0) == 2
+    assert call(w=FAKE + 4) == 3 and call(out=FAKE + 8) == 3
+    assert call(scratch=0) == 4
+
+
+def test_ternary_code_by_comparison_is_the_rounded_quotient():
+    """clip(rne(w / s), -1, 1) in float32 is 1 exactly where w > 0.5 s (what
+    the one-pass load compares), around half the scale to the last bit."""
+    rng = np.random.default_rng(7)
+    for i in range(200):
+        s = np.float32(np.exp(rng.uniform(-11, 30)))
+        if i % 3 == 0:
+            s = np.nextafter(np.float32(2.0 ** int(rng.integers(-16, 20))), np.float32(0))
+        t = np.float32(0.5) * s
+        near = t.view(np.uint32) + np.arange(-50, 51, dtype=np.int64)
+        w = np.concatenate([near.astype(np.uint32).view(np.float32), rng.standard_normal(500).astype(np.float32) * s])
+        w = np.concatenate([w, -w])
+        q = np.clip(np.round(w / s), -1, 1)
+        assert np.array_equal(q, (w > t).astype(int) - (~(w >= -t)).astype(int))

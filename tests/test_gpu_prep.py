@@ -73,3 +73,44 @@ def test_repack_matches_oracle_layout(orc, k, n):
     got = wdev.cpu().numpy().view(np.uint32)
     assert np.array_equal(got, orc.devlayout_encode(w_kn))
     assert np.array_equal(orc.devlayout_decode(got, k, n), w_kn)
+
+
+@pytest.mark.parametrize("n", [1, 7, 8, 9, 127, 128, 129, 135, 136, 137, 263, 1031, 4103, 6000, 8184, 8191, 8193, 16383])
+def test_weight_scale_of_every_block_length(orc, n):
+    """Partial blocks around the leaves of numpy's split tree, aligned and not:
+    the scale is numpy's to the bit."""
+    w = H.latent(1, n + 1, seed=43 + n).reshape(-1)
+    d = H.to_dev(w)
+    for view, host in ((d[:n], w[:n]), (d[1:], w[1:])):
+        q_d, s_d = Q.weight_quant_ternary(view)
+        q_h, s_h = orc.weight_quant_ternary(np.ascontiguousarray(host))
+        assert np.float32(s_d) == s_h and np.array_equal(q_d.cpu().numpy(), q_h)
+
+
+@pytest.mark.parametrize("n,k,special", [(32, 32, False), (64, 96, False), (96, 160, True), (160, 128, True),
+                                         (2560, 6912, False), (1440, 4064, True)])
+def test_quantize_for_gemm_matches_the_three_passes(orc, n, k, special):
+    """The one-pass load against quantise, tiles and repack, bit for bit; with
+    `special`, ties at half the scale, zeros, a NaN (the scale is then eps) and,
+    in a second weight, an infinity (an infinite scale)."""
+    from bitnet_tt.kernels.pack import pack_ternary_tilized_device, quantize_for_gemm, repack_for_gemm
+
+    print(f"quantize_for_gemm {n}x{k}", flush=True)
+    w = H.latent(n, k, seed=n + k)
+    ws = [w]
+    if special:
+        t = np.float32(0.5) * np.mean(np.abs(w), dtype=np.float32)
+        w2, w3, w4 = w.copy(), w.copy(), w.copy()
+        w2[::3, ::5] = t
+        w2[1::3, ::7] = np.nextafter(-t, np.float32(-1))
+        w2[2, :] = 0.0
+        w3[0, 0] = np.nan
+        w3[3, 1:9] = [5e-6, -5e-6, 5.1e-6, -5.1e-6, 0.0, 1.0, -0.0, np.nan]
+        w4[n // 2, k // 2] = -np.inf
+        ws += [w2, w3, w4]
+    for x in ws:
+        d = H.to_dev(x)
+        q, s = Q.weight_quant_ternary(d)
+        ref = repack_for_gemm(pack_ternary_tilized_device(q), k, n)
+        got, s2 = quantize_for_gemm(d)
+        assert s == s2 and torch.equal(got, ref)
