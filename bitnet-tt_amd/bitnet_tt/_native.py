@@ -10,8 +10,10 @@ calls are stream-ordered and can be recorded into a HIP graph.
 from __future__ import annotations
 
 import ctypes
+import itertools
 import os
 import threading
+import weakref
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 # BTL_LIBRARY names another build of the same library (the host-sanitizer
@@ -185,10 +187,30 @@ def require_cuda(t, name: str) -> None:
         raise ValueError(f"{name} must be contiguous")
 
 
+def _resolve_raw_stream():
+    """current_stream(index).cuda_stream without the Stream object around it
+    (1.7 us a call) where this torch has it."""
+    import torch
+
+    global _raw_stream
+    _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (
+        lambda index: torch.cuda.current_stream(index).cuda_stream)
+    return _raw_stream
+
+
+_raw_stream = None
+
+
+def raw_stream(index: int) -> int:
+    """Handle of the calling thread's current stream on device ``index``."""
+    return (_raw_stream or _resolve_raw_stream())(index)
+
+
 def stream_of(device) -> ctypes.c_void_p:
     import torch
 
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    d = torch.device(device)
+    return ctypes.c_void_p(raw_stream(torch.cuda.current_device() if d.index is None else d.index))
 
 
 def segments_arrays(scales, ends):
@@ -203,15 +225,59 @@ def segments_arrays(scales, ends):
 
 # Per (device, stream) workspace.  Calls on one stream are ordered, so they
 # can share it; the activation kernel of every fused call clears the split-K
-# counters it uses.
+# counters it uses.  A workspace that holds one object's prepared state (the
+# decode step's weight table) is that object's own on each stream: its key
+# ends with the object's owner_id(), and it goes when the object does.
 _workspaces: dict = {}
+# workspace_ptr's lookups: (kind, device index, stream, error offset, owner) ->
+# (address, bytes, buffer).  Emptied whenever a workspace is made or released.
+_fast: dict = {}
+_owner_ids = itertools.count(1)
+_owners: "weakref.WeakKeyDictionary" = weakref.WeakKeyDictionary()
 
 
-def has_workspace(device, nbytes: int, kind: str = "bitlinear") -> bool:
+def owner_id(obj) -> int:
+    """The number of ``obj`` whose workspaces are released with it (a copy of
+    ``obj`` gets its own)."""
+    n = _owners.get(obj)
+    if n is None:
+        n = _owners.setdefault(obj, next(_owner_ids))
+        weakref.finalize(obj, _release_owner, n).atexit = False
+    return n
+
+
+def _release_owner(n: int) -> None:
+    _fast.clear()
+    for key in [k for k in list(_workspaces) if len(k) == 4 and k[3] == n]:
+        buf = _workspaces.pop(key, None)
+        _error_words.pop(key, None)
+        if buf is not None:
+            _prepared_for.pop(buf.data_ptr(), None)
+            _reset_hooks.pop(buf.data_ptr(), None)
+
+
+def workspace_ptr(index: int, nbytes: int, kind: str, error_offset: int, stream: int, owner: int = 0):
+    """(address, bytes) of :func:`workspace` on device ``index`` and the current
+    stream, whose handle is ``stream``."""
+    key = (kind, index, stream, error_offset, owner)
+    hit = _fast.get(key)
+    if hit is None or hit[1] < nbytes:
+        import torch
+
+        buf = workspace(torch.device("cuda", index), nbytes, kind, error_offset, owner)
+        hit = _fast[key] = (buf.data_ptr(), buf.numel(), buf)
+    return hit
+
+
+def _key(kind: str, device, stream: int, owner: int) -> tuple:
+    return (kind, _device_key(device), stream) + ((owner,) if owner else ())
+
+
+def has_workspace(device, nbytes: int, kind: str = "bitlinear", owner: int = 0) -> bool:
     """True when the current stream already owns a workspace of nbytes."""
     import torch
 
-    buf = _workspaces.get((kind, _device_key(device), torch.cuda.current_stream(device).cuda_stream))
+    buf = _workspaces.get(_key(kind, device, torch.cuda.current_stream(device).cuda_stream, owner))
     return buf is not None and buf.numel() >= nbytes
 
 
@@ -250,21 +316,22 @@ def _device_key(device) -> str:
     return str(d)
 
 
-def workspace(device, nbytes: int, kind: str = "bitlinear", error_offset: int | None = None):
+def workspace(device, nbytes: int, kind: str = "bitlinear", error_offset: int | None = None, owner: int = 0):
     """Zero-filled device workspace of at least nbytes for the current stream.
 
     kind separates workspaces whose layouts differ ("bitlinear" for
     btl_bitlinear_fused / btl_gemm_i8t2, "step" for btl_decode_step).  A
     workspace that grows is replaced by a fresh zero-filled one; the old one
     is released in stream order, after the calls that used it.
-    ``error_offset`` registers the byte offset of a sticky error word inside
+    ``owner`` (owner_id) makes it one object's own.  ``error_offset`` registers the byte offset of a sticky error word inside
     the workspace, which :func:`check_errors` reads."""
     import torch
 
     stream = torch.cuda.current_stream(device)
-    key = (kind, _device_key(device), stream.cuda_stream)
+    key = _key(kind, device, stream.cuda_stream, owner)
     buf = _workspaces.get(key)
     if buf is None or buf.numel() < nbytes:
+        _fast.clear()
         if buf is not None:
             _prepared_for.pop(buf.data_ptr(), None)
             _reset_hooks.pop(buf.data_ptr(), None)

@@ -258,6 +258,13 @@ class BitLinearDecodeStep:
         self.attn_out = acts(qd)
         self.qkv_out = torch.empty((B, c.qkv_dim), dtype=torch.bfloat16, device=self.device)
         self.ffn_h = torch.empty((B, c.intermediate_size), dtype=torch.bfloat16, device=self.device)
+        # the one-launch step's workspace on this stream, with the buffers and
+        # not in the first step (0 bytes: a shape that only step_per_call takes)
+        L = N.lib()
+        nbytes = int(L.btl_decode_step_workspace_bytes(B, c.hidden_size, c.intermediate_size, c.qkv_dim,
+                                                       len(self.layers)))
+        if nbytes > 0 and qd == c.hidden_size:
+            N.workspace(self.hidden.device, nbytes, "step", int(L.btl_decode_step_error_offset()), N.owner_id(self))
         return self
 
     def reset_hidden(self):
@@ -346,10 +353,11 @@ class BitLinearDecodeStep:
         return self._st
 
     def _step_workspace(self, attention: bool):
-        """This stream's workspace of the one-launch step, prepared for the
-        weight table (and, with ``attention``, for the KV-cache table) by
-        synchronous copies: the first call on a stream must come before a
-        graph capture."""
+        """(address, bytes, stream) of this object's workspace of the one-launch
+        step on the current stream, prepared for the weight table (and, with
+        ``attention``, for the KV-cache table) by synchronous copies: the first
+        call on a stream must come before a graph capture.  Each object has its
+        own, so that models taking turns on a stream stay prepared."""
         import ctypes
 
         import torch
@@ -363,40 +371,42 @@ class BitLinearDecodeStep:
         L = N.lib()
         table = self._step_table()
         dev = self.hidden.device
+        stream = N.raw_stream(dev.index)
+        owner = N.owner_id(self)
         nbytes = int(L.btl_decode_step_workspace_bytes(B, H, F, c.qkv_dim, nl))
         capturing = torch.cuda.is_current_stream_capturing()
-        if capturing and not N.has_workspace(dev, nbytes, "step"):
+        if capturing and not N.has_workspace(dev, nbytes, "step", owner):
             raise RuntimeError("run one eager decode step on this stream before capturing it in a graph")
-        ws = N.workspace(dev, nbytes, kind="step", error_offset=int(L.btl_decode_step_error_offset()))
+        ptr, ws_bytes, ws = N.workspace_ptr(dev.index, nbytes, "step", int(L.btl_decode_step_error_offset()), stream,
+                                            owner)
         caches = None
         if attention:
             if getattr(self, "kv", None) is None:
                 raise RuntimeError("step_persistent_full needs alloc_attention() first")
-            caches = tuple((kv.key_cache.data_ptr(), kv.value_cache.data_ptr()) for kv in self.kv)
+            caches = tuple([(kv.key_cache.data_ptr(), kv.value_cache.data_ptr()) for kv in self.kv])
         ready = getattr(self, "_ws_caches", {})
         self._ws_caches = ready
-        if N.workspace_prepared_for(ws) is not table or (attention and ready.get(ws.data_ptr()) != caches):
+        if N.workspace_prepared_for(ws) is not table or (attention and ready.get(ptr) != caches):
             if capturing:
                 raise RuntimeError("run one eager decode step on this stream before capturing it in a graph")
             torch.cuda.current_stream(dev).synchronize()  # earlier launches on this workspace are done
 
             def prepare():
-                N.check(L.btl_decode_step_prepare(B, H, F, c.qkv_dim, nl, table, N.ptr(ws), ws.numel()),
+                N.check(L.btl_decode_step_prepare(B, H, F, c.qkv_dim, nl, table, ptr, ws_bytes),
                         "btl_decode_step_prepare")
                 N.set_workspace_prepared_for(ws, table)
-                cached = ready.get(ws.data_ptr())
+                cached = ready.get(ptr)
                 if cached is not None:
                     kp = (ctypes.c_void_p * nl)(*[k for k, _ in cached])
                     vp = (ctypes.c_void_p * nl)(*[v for _, v in cached])
-                    N.check(L.btl_decode_step_attention_prepare(B, H, F, c.qkv_dim, nl, kp, vp, N.ptr(ws),
-                                                                ws.numel()),
+                    N.check(L.btl_decode_step_attention_prepare(B, H, F, c.qkv_dim, nl, kp, vp, ptr, ws_bytes),
                             "btl_decode_step_attention_prepare")
 
             if attention:
-                ready[ws.data_ptr()] = caches
+                ready[ptr] = caches
             prepare()
             N.set_workspace_reset(ws, prepare)
-        return ws
+        return ptr, ws_bytes, stream
 
     def step_persistent(self):
         """The whole step's BitLinears as one btl_decode_step launch (every
@@ -411,12 +421,10 @@ class BitLinearDecodeStep:
         for t, name in ((self.hidden, "hidden"), (self.attn_out, "attn_out"), (self.qkv_out, "qkv_out"),
                         (self.ffn_h, "ffn_h")):
             N.require_cuda(t, name)
-        ws = self._step_workspace(attention=False)
-        L = N.lib()
-        dev = self.hidden.device
+        ws, ws_bytes, stream = self._step_workspace(attention=False)
         N.check(
-            L.btl_decode_step(B, H, F, c.qkv_dim, nl, float(self.eps), N.ptr(self.attn_out), N.ptr(self.hidden),
-                              N.ptr(self.qkv_out), N.ptr(self.ffn_h), N.ptr(ws), ws.numel(), N.stream_of(dev)),
+            N.lib().btl_decode_step(B, H, F, c.qkv_dim, nl, float(self.eps), N.ptr(self.attn_out), N.ptr(self.hidden),
+                                    N.ptr(self.qkv_out), N.ptr(self.ffn_h), ws, ws_bytes, stream),
             "btl_decode_step",
         )
         return self.hidden
@@ -436,16 +444,14 @@ class BitLinearDecodeStep:
         for t, name in ((self.hidden, "hidden"), (self.attn_out, "attn_out"), (self.qkv_out, "qkv_out"),
                         (self.ffn_h, "ffn_h")):
             N.require_cuda(t, name)
-        ws = self._step_workspace(attention=True)
+        ws, ws_bytes, stream = self._step_workspace(attention=True)
         att = self.attention
-        L = N.lib()
-        dev = self.hidden.device
         N.check(
-            L.btl_decode_step_full(B, H, F, c.qkv_dim, nl, float(self.eps), att.num_kv_heads, att.max_seq_len,
-                                   N.ptr(self.pos), N.ptr(att.rope_cos), N.ptr(att.rope_sin),
-                                   int(att.use_fused_rope), float(att.scale), N.ptr(self.hidden),
-                                   N.ptr(self.qkv_out), N.ptr(self.attn_out), N.ptr(self.ffn_h), N.ptr(ws),
-                                   ws.numel(), N.stream_of(dev)),
+            N.lib().btl_decode_step_full(B, H, F, c.qkv_dim, nl, float(self.eps), att.num_kv_heads, att.max_seq_len,
+                                         N.ptr(self.pos), N.ptr(att.rope_cos), N.ptr(att.rope_sin),
+                                         int(att.use_fused_rope), float(att.scale), N.ptr(self.hidden),
+                                         N.ptr(self.qkv_out), N.ptr(self.attn_out), N.ptr(self.ffn_h), ws, ws_bytes,
+                                         stream),
             "btl_decode_step_full",
         )
         return self.hidden
@@ -463,9 +469,9 @@ class BitLinearDecodeStep:
         nbytes = int(L.btl_decode_step_workspace_bytes(B, H, F, c.qkv_dim, nl))
         import torch
 
-        if torch.cuda.is_current_stream_capturing() and not N.has_workspace(dev, nbytes, "step"):
+        if torch.cuda.is_current_stream_capturing() and not N.has_workspace(dev, nbytes, "step", N.owner_id(self)):
             raise RuntimeError("run one eager decode step on this stream before capturing it in a graph")
-        ws = N.workspace(dev, nbytes, kind="step", error_offset=int(L.btl_decode_step_error_offset()))
+        ws = N.workspace(dev, nbytes, "step", int(L.btl_decode_step_error_offset()), N.owner_id(self))
         N.check(L.btl_decode_step_floor(B, H, F, c.qkv_dim, nl, N.ptr(ws), ws.numel(), N.stream_of(dev)),
                 "btl_decode_step_floor")
 

@@ -20,8 +20,11 @@ absorbed by attn_sub_norm, attention.py:817-839).
 
 from __future__ import annotations
 
+import functools
+
 import numpy as np
 
+from .. import _native as N
 from .bitlinear import Linear, quantize_and_transpose_weight
 
 
@@ -88,6 +91,14 @@ class QKVProjection:
         return self.qkv(hidden, norm_weight=norm_weight, norm_epsilon=norm_epsilon)
 
 
+@functools.lru_cache(maxsize=4096)
+def _attention_bytes(index: int, b: int, h: int, hkv: int, s: int) -> tuple[int, int]:
+    """(workspace bytes, error word offset) of an attention call on device ``index``."""
+    L = N.lib()
+    return (int(L.btl_decode_attention_workspace_bytes(b, h, hkv, s)),
+            int(L.btl_decode_attention_error_offset(b, hkv)))
+
+
 class KVCache:
     """Pre-allocated per-layer cache (attention.py KVCache): key_cache and
     value_cache [batch, kv_heads, max_seq_len, head_dim] bf16."""
@@ -143,8 +154,6 @@ class DecodeAttention:
         returns bf16 [B, H D] (written into ``out`` when given)."""
         import torch
 
-        from .. import _native as N
-
         B = qkv.shape[0]
         H, Hkv, D, S = self.num_heads, self.num_kv_heads, self.head_dim, self.max_seq_len
         N.require_cuda(qkv, "qkv")
@@ -157,34 +166,29 @@ class DecodeAttention:
             raise ValueError("cache shape does not match")
         if out is None:
             out = torch.empty((B, H * D), dtype=torch.bfloat16, device=qkv.device)
-        L = N.lib()
-        nbytes = int(L.btl_decode_attention_workspace_bytes(B, H, Hkv, S))
+        index = qkv.device.index
+        stream = N.raw_stream(index)
+        nbytes, off = _attention_bytes(index, B, H, Hkv, S)
         if torch.cuda.is_current_stream_capturing() and not N.has_workspace(qkv.device, nbytes, "attention"):
             raise RuntimeError("run one eager attention call on this stream before capturing it in a graph")
-        ws = N.workspace(qkv.device, nbytes, kind="attention",
-                         error_offset=int(L.btl_decode_attention_error_offset(B, Hkv)))
-        N.check(
-            L.btl_decode_attention(N.ptr(qkv), B, H, Hkv, D, S, N.ptr(pos), N.ptr(self.rope_cos), N.ptr(self.rope_sin),
-                                   int(self.use_fused_rope), float(self.scale), N.ptr(kv_cache.key_cache),
-                                   N.ptr(kv_cache.value_cache), N.ptr(out), N.ptr(ws), ws.numel(),
-                                   N.stream_of(qkv.device)),
-            "btl_decode_attention",
-        )
+        ws, ws_bytes, _ = N.workspace_ptr(index, nbytes, "attention", off, stream)
+        rc = N.lib().btl_decode_attention(
+            qkv.data_ptr(), B, H, Hkv, D, S, pos.data_ptr(), self.rope_cos.data_ptr(), self.rope_sin.data_ptr(),
+            int(self.use_fused_rope), float(self.scale), kv_cache.key_cache.data_ptr(),
+            kv_cache.value_cache.data_ptr(), out.data_ptr(), ws, ws_bytes, stream)
+        if rc != N.BTL_OK:
+            N.check(rc, "btl_decode_attention")
         return out
 
     def check(self) -> None:
         """Raise RuntimeError if a call since the last check met a position
         outside [0, max_seq_len) (or any other launch on the device reported
         a timed-out wait); synchronises the device."""
-        from .. import _native as N
-
         N.check_errors(self.device)
 
     def error_word(self, device=None, B: int = 32) -> int:
         """Non-zero once a position outside [0, max_seq_len) reached a call on
         the current stream."""
-        from .. import _native as N
-
         L = N.lib()
         ws = N.workspace(self.device if device is None else device, 0, kind="attention")
         off = int(L.btl_decode_attention_error_offset(B, self.num_kv_heads))

@@ -76,16 +76,17 @@ class LMHead:
             torch.empty((M, V), dtype=torch.float32, device=hidden.device) if return_logits else None)
         tokens = tokens_out if tokens_out is not None else torch.empty(M, dtype=torch.int32, device=hidden.device)
         L = N.lib()
-        stream = N.stream_of(hidden.device)
+        index = hidden.device.index
+        stream = N.raw_stream(index)
         nbytes = int(L.btl_lm_head_workspace_bytes())
         if torch.cuda.is_current_stream_capturing() and not N.has_workspace(hidden.device, nbytes, "lm_head"):
             # a workspace made inside a capture would be re-zeroed by every replay
             raise RuntimeError("run one eager head call on this stream before capturing it in a graph")
-        ws = N.workspace(hidden.device, nbytes, kind="lm_head")
-        N.check(L.btl_rmsnorm(N.ptr(x), M, H, H, N.ptr(self.norm_weight), float(self.eps), N.ptr(xn), stream),
+        ws, ws_bytes, _ = N.workspace_ptr(index, nbytes, "lm_head", None, stream)
+        N.check(L.btl_rmsnorm(x.data_ptr(), M, H, H, N.ptr(self.norm_weight), float(self.eps), xn.data_ptr(), stream),
                 "btl_rmsnorm")
-        N.check(L.btl_lm_head(N.ptr(xn), M, H, V, N.ptr(self.weight), N.ptr(logits) if logits is not None else None,
-                              N.ptr(tokens), N.ptr(ws), ws.numel(), stream), "btl_lm_head")
+        N.check(L.btl_lm_head(xn.data_ptr(), M, H, V, self.weight.data_ptr(), N.ptr(logits), tokens.data_ptr(), ws,
+                              ws_bytes, stream), "btl_lm_head")
         return logits, tokens
 
     def weight_bytes(self) -> int:

@@ -18,6 +18,7 @@ backend: inputs must live on a ROCm device and libbtl.so must be built.
 
 from __future__ import annotations
 
+import functools
 import os
 from dataclasses import dataclass, field
 
@@ -140,6 +141,17 @@ def ternary_matmul(
     return out
 
 
+# The library reads these arrays during the call and never writes them.
+_segments = functools.lru_cache(maxsize=4096)(N.segments_arrays)
+
+
+@functools.lru_cache(maxsize=4096)
+def _fused_bytes(index: int, m: int, k: int, n: int, epi: int, splitk: int) -> tuple[int, int]:
+    """(workspace bytes, error word offset) of a fused call on device ``index``."""
+    L = N.lib()
+    return int(L.btl_fused_workspace_bytes(m, k, n, epi, splitk)), int(L.btl_fused_error_offset())
+
+
 def check(device=None) -> None:
     """Raise RuntimeError if a bounded wait of a fused decode launch on
     ``device`` ran out since the last check (the launch then returned invalid
@@ -173,51 +185,55 @@ def ternary_matmul_into(
     Nf = w.out_features
     M = x.numel() // K
     epi = EPILOGUES[epilogue]
-    for t, name in ((x, "x"), (out, "out"), (residual, "residual"), (acc_out, "acc_out"), (xq_out, "xq_out")):
-        N.require_cuda(t, name)
+    N.require_cuda(x, "x")
+    N.require_cuda(out, "out")
     if out.dtype != torch.bfloat16:
         raise ValueError("out must be bfloat16")
     n_out = Nf // 2 if epi == N.EPI_RELU2_MUL else Nf
     if out.numel() != M * n_out:
         raise ValueError(f"out has {out.numel()} elements, expected {M}x{n_out}")
-    if residual is not None and (residual.numel() != M * n_out or residual.dtype != torch.bfloat16):
-        raise ValueError("residual must be bf16 with the output's shape")
-    if acc_out is not None and (acc_out.dtype != torch.int32 or acc_out.numel() != M * Nf):
-        raise ValueError("acc_out must be int32 [M, N]")
-    if xq_out is not None and (xq_out.dtype != torch.int8 or xq_out.numel() != M * K):
-        raise ValueError("xq_out must be int8 [M, K]")
-    gamma = None
+    gamma = res = acc = xq = None  # addresses
     eps = 0.0
+    if residual is not None:
+        N.require_cuda(residual, "residual")
+        if residual.numel() != M * n_out or residual.dtype != torch.bfloat16:
+            raise ValueError("residual must be bf16 with the output's shape")
+        res = residual.data_ptr()
+    if acc_out is not None:
+        N.require_cuda(acc_out, "acc_out")
+        if acc_out.dtype != torch.int32 or acc_out.numel() != M * Nf:
+            raise ValueError("acc_out must be int32 [M, N]")
+        acc = acc_out.data_ptr()
+    if xq_out is not None:
+        N.require_cuda(xq_out, "xq_out")
+        if xq_out.dtype != torch.int8 or xq_out.numel() != M * K:
+            raise ValueError("xq_out must be int8 [M, K]")
+        xq = xq_out.data_ptr()
     if norm_weight is not None:
         if norm_epsilon is None:
             raise ValueError("norm_weight needs norm_epsilon")
-        gamma = norm_weight
-        N.require_cuda(gamma, "norm_weight")
-        if gamma.dtype != torch.bfloat16 or gamma.numel() != K:
+        N.require_cuda(norm_weight, "norm_weight")
+        if norm_weight.dtype != torch.bfloat16 or norm_weight.numel() != K:
             raise ValueError("norm_weight must be bf16 with K elements")
+        gamma = norm_weight.data_ptr()
         eps = float(norm_epsilon)
     if weight_scale is None:
-        scales = tuple(w.segment_scales)
-        ends = tuple(w.segment_ends)
+        sc, en, nseg = _segments(tuple(w.segment_scales), tuple(w.segment_ends))
     elif isinstance(weight_scale, (int, float)):
-        scales, ends = (float(weight_scale),), (Nf,)
+        sc, en, nseg = N.segments_arrays((float(weight_scale),), (Nf,))
     else:
         scales = tuple(float(s) for s in weight_scale)
-        ends = tuple(w.segment_ends)
-        if len(scales) != len(ends):
+        if len(scales) != len(w.segment_ends):
             raise ValueError("weight_scale needs one value per weight segment")
-    sc, en, nseg = N.segments_arrays(scales, ends)
-    L = N.lib()
-    dev = x.device
-    ws_bytes = int(L.btl_fused_workspace_bytes(M, K, Nf, epi, splitk))
-    ws = N.workspace(dev, ws_bytes, error_offset=int(L.btl_fused_error_offset()))
-    N.check(
-        L.btl_bitlinear_fused(
-            N.ptr(x), M, K, K, N.ptr(gamma), eps, N.ptr(w.data), Nf, sc, en, nseg, epi, N.ptr(residual),
-            N.ptr(out), N.ptr(acc_out), N.ptr(xq_out), N.ptr(ws), ws.numel(), int(splitk), N.stream_of(dev),
-        ),
-        "btl_bitlinear_fused",
-    )
+        sc, en, nseg = N.segments_arrays(scales, tuple(w.segment_ends))
+    index = x.device.index
+    stream = N.raw_stream(index)
+    nbytes, off = _fused_bytes(index, M, K, Nf, epi, splitk)
+    ws, ws_bytes, _ = N.workspace_ptr(index, nbytes, "bitlinear", off, stream)
+    rc = N.lib().btl_bitlinear_fused(x.data_ptr(), M, K, K, gamma, eps, w.data.data_ptr(), Nf, sc, en, nseg, epi, res,
+                                     out.data_ptr(), acc, xq, ws, ws_bytes, splitk, stream)
+    if rc != N.BTL_OK:
+        N.check(rc, "btl_bitlinear_fused")
     if _check_after_call if check_errors is None else check_errors:
-        N.check_errors(dev)
+        N.check_errors(x.device)
     return out

@@ -442,3 +442,48 @@ def test_c4_persistent_step_many_replays(orc, c4_model):
             print(f"persistent step replay {rep + 1}", flush=True)
     step.check()
     assert not bad, f"replays {bad[:10]} differ from the oracle chain"
+
+
+def test_models_taking_turns_keep_their_own_step_workspace(orc):
+    """Two models' one-launch steps in turn on one stream, with graph replays of
+    the first between them, give what each gives alone; a model's workspaces
+    go with it."""
+    import gc
+
+    from bitnet_tt import _native as N
+    from bitnet_tt.config import BitNetMiniConfig
+    from bitnet_tt.decode import BitLinearDecodeStep
+
+    cfg = BitNetMiniConfig(num_layers=2, num_attention_heads=2)
+    print("two models in turn", flush=True)
+    models = [BitLinearDecodeStep.random_init(cfg, H.dev(), seed=61 + i, batch=8 + i).alloc_buffers(seed=71 + i)
+              for i in range(2)]
+    refs = []
+    for m in models:
+        m.step_per_call()
+        refs.append(m.hidden.clone())
+        m.reset_hidden()
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(s):
+        for m in models:
+            m.step_persistent()
+    s.synchronize()
+    with torch.cuda.graph(g, stream=s):
+        models[0].step_persistent()
+    for rep in range(3):
+        for m, ref in zip(models, refs):
+            m.reset_hidden()
+            m.step_persistent()
+            assert torch.equal(m.hidden, ref)
+        models[0].reset_hidden()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(models[0].hidden, refs[0])
+        m.check()
+    owners = [N.owner_id(m) for m in models]
+    assert {k[3] for k in N._workspaces if len(k) == 4} >= set(owners)
+    del g, m, models
+    gc.collect()
+    assert not {k[3] for k in N._workspaces if len(k) == 4} & set(owners)
