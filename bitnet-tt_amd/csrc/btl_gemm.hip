@@ -29,7 +29,8 @@
 // so weight streaming overlaps the prologue and a launch is saved.
 //
 // Prefill (M > 32): 128x256 output tiles, operands staged through LDS once
-// per superblock and shared by the four waves (64x128 each).
+// per superblock and shared by the four waves (64x128 each); wide tiles; and,
+// for few rows, workgroups of the decode kind (k_gemm_rows).
 #include <stdlib.h>
 
 #include <atomic>
@@ -1206,6 +1207,160 @@ __global__ __launch_bounds__(256, 2) void k_gemm_wide(GemmArgs p, int ngm, int n
   BTL_TRACE_AT(14);
 }
 
+// ------------------------------------------- prefill, few row blocks ----
+// Short prompts (a few row blocks of 32) of the fused BitLinear: the decode
+// body's shape with more rows.  A workgroup of eight waves owns RB = RBW * RH row blocks x TPW column
+// tiles (relu2: a gate tile and its up tile) and all of K; RH waves share each
+// K slice, each on RBW row blocks, and KW = 8 / RH split the superblocks.
+// Operands go from global memory straight to the MFMA registers, D superblocks
+// ahead, with no barrier in the loop; the partial sums meet in LDS once.  The
+// 64-row tiles of k_gemm_prefill are too few to fill the chip here, and the
+// split-K that makes up for it moves a 64 KiB partial per workgroup through
+// memory.  One round of workgroups is bound by the latency of its loads, more
+// by the operands through a CU's L1 (32 rows x 64 columns of K = 2560: 120 KB,
+// 1.9 us).  With two tiles D = 1 beat D = 2 and 3 (2560 ->
+// 3840, M = 512: 10.3 against 11.0 and 11.8 us): the second workgroup of the CU
+// hides the wait.  One row block a wave beat two (5.0 against 9.3 us there at
+// M = 100), and 32 rows x 4 tiles was 12.0.
+template <int RBW, int RH, int TPW, int D, int EPI>
+__global__ __launch_bounds__(512) void k_gemm_rows(GemmArgs p, int ngm, int ngn) {
+  constexpr int KW = 8 / RH, RB = RBW * RH;
+  constexpr int OT = EPI == EPI_RELU2 ? TPW / 2 : TPW;  // output tiles
+  static_assert(EPI == EPI_SCALE || TPW % 2 == 0, "relu2 pairs gate tiles with their up tiles");
+  __shared__ __attribute__((aligned(16))) int32_t red[KW][RB][TPW][16][64];
+  __shared__ float s_adq[RB * 32];
+  __shared__ int32_t s_rs[RB * 32];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), kw = wv % KW, rh = wv / KW;
+  // XCD x takes a contiguous range of column groups, row groups inner: the
+  // row groups of a column group share its weights in one L2
+  const int nwg = ngm * ngn, per = (nwg + kPfXcds - 1) / kPfXcds;
+  const int wg = (int)(blockIdx.x % kPfXcds) * per + (int)(blockIdx.x / kPfXcds);
+  if (wg >= nwg) return;
+  const int gm = wg % ngm, gn = wg / ngm;
+  const int KS = p.KS;
+  int tile[TPW];
+#pragma unroll
+  for (int t = 0; t < TPW; ++t)  // relu2: the gate tiles, then their up tiles
+    tile[t] = EPI == EPI_RELU2 ? (t / OT) * (p.NT >> 1) + min(gn * OT + t % OT, (p.NT >> 1) - 1)
+                               : min(gn * TPW + t, p.NT - 1);
+  const int wb = kw * KS / KW, we = (kw + 1) * KS / KW;
+
+  const int8_t* pa[RBW];
+#pragma unroll
+  for (int x = 0; x < RBW; ++x) pa[x] = p.xa + (int64_t)min(gm * RB + rh * RBW + x, p.Mb - 1) * KS * 4096;
+  const int8_t* pb[TPW];
+#pragma unroll
+  for (int t = 0; t < TPW; ++t) pb[t] = reinterpret_cast<const int8_t*>(p.wdev) + (int64_t)tile[t] * KS * 1024;
+  v4i a[D][RBW][4], b[D][TPW];
+  // Every slot of the pipeline is loaded on every pass, one past the slice
+  // from a single line: each wait then counts exactly the loads it needs.
+  auto load = [&](int j, int sb) {
+    const bool in = sb < we;
+    const int s = in ? sb : 0, lo = in ? lane * 16 : 0;
+#pragma unroll
+    for (int x = 0; x < RBW; ++x)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) a[j][x][q] = ld128(pa[x] + s * 4096 + q * 1024 + lo);
+#pragma unroll
+    for (int t = 0; t < TPW; ++t) b[j][t] = ld128(pb[t] + s * 1024 + lo);
+  };
+  v16i acc[RBW][TPW];
+#pragma unroll
+  for (int x = 0; x < RBW; ++x)
+#pragma unroll
+    for (int t = 0; t < TPW; ++t) acc[x][t] = (v16i){0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+  for (int j = 0; j < D; ++j) load(j, wb + j);
+  if (tid < RB * 32) {
+    const int row = gm * RB * 32 + tid;
+    s_adq[tid] = p.a_dq[min(row, p.Mb * 32 - 1)];
+    s_rs[tid] = p.rowsum[min(row, p.M - 1)];  // rows past M are not stored
+  }
+  for (int base = wb; base < we; base += D) {
+#pragma unroll
+    for (int j = 0; j < D; ++j) {
+      if (base + j < we) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+          for (int t = 0; t < TPW; ++t) {
+            const v4i bb = unpack_b((uint32_t)b[j][t][q]);
+#pragma unroll
+            for (int x = 0; x < RBW; ++x)
+              acc[x][t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[j][x][q], bb, acc[x][t], 0, 0, 0);
+          }
+      }
+      load(j, base + j + D);
+    }
+  }
+#pragma unroll
+  for (int x = 0; x < RBW; ++x)
+#pragma unroll
+    for (int t = 0; t < TPW; ++t)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) red[kw][rh * RBW + x][t][r][lane] = acc[x][t][r];
+  __syncthreads();
+  // Each thread finishes 8 consecutive columns of a row, one 16-byte store.
+  constexpr int CPR = OT * 4, CHUNKS = RB * 32 * CPR;
+#pragma unroll
+  for (int c0 = 0; c0 < CHUNKS; c0 += 512) {
+    const int c = c0 + tid;
+    if (CHUNKS % 512 != 0 && c >= CHUNKS) break;
+    const int il = c / CPR, t = (c % CPR) >> 2, jq = c & 3;
+    const int i = gm * RB * 32 + il;
+    const int ot = gn * OT + t, up = ot + (p.NT >> 1);  // output (and gate) tile, its up tile
+    if (i >= p.M || ot >= (EPI == EPI_RELU2 ? p.NT >> 1 : p.NT)) continue;
+    const int64_t at = (int64_t)i * p.n_out + ot * 32 + jq * 8;
+    uint4 res = make_uint4(0u, 0u, 0u, 0u);
+    if (EPI == EPI_SCALE && p.residual) res = *reinterpret_cast<const uint4*>(p.residual + at);
+    const int rb = il >> 5, r = il & 31;
+    // row r of a block: lane half (r >> 2) & 1, register 4 (r >> 3) + (r & 3)
+    const int reg = ((r >> 3) << 2) | (r & 3), l0 = ((r >> 2) & 1) * 32 + jq * 8;
+    const int32_t rs = s_rs[il];
+    const float ad = s_adq[il];
+    int32_t e[EPI == EPI_RELU2 ? 2 : 1][8];
+#pragma unroll
+    for (int u = 0; u < (EPI == EPI_RELU2 ? 2 : 1); ++u) {
+#pragma unroll
+      for (int k = 0; k < 8; ++k) e[u][k] = -rs;
+#pragma unroll
+      for (int w = 0; w < KW; ++w) {
+        const v4i v0 = *reinterpret_cast<const v4i*>(&red[w][rb][u * OT + t][reg][l0]);
+        const v4i v1 = *reinterpret_cast<const v4i*>(&red[w][rb][u * OT + t][reg][l0 + 4]);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) e[u][k] += v0[k], e[u][4 + k] += v1[k];
+      }
+      if (p.acc_out) {
+        int32_t* const ao = p.acc_out + (int64_t)i * p.N + (u ? up : ot) * 32 + jq * 8;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) ao[k] = e[u][k];
+      }
+    }
+    uint32_t o[4];
+    const float f = seg_scale_of(p, ot * 32) * ad;
+    if constexpr (EPI == EPI_RELU2) {
+      const float fu = seg_scale_of(p, up * 32) * ad;
+#pragma unroll
+      for (int h = 0; h < 4; ++h) {
+        const uint32_t g2 = f2bf_pair((float)e[0][2 * h] * f, (float)e[0][2 * h + 1] * f);
+        const uint32_t u2 = f2bf_pair((float)e[1][2 * h] * fu, (float)e[1][2 * h + 1] * fu);
+        const float g0 = bf_lo(g2) > 0.0f ? bf_lo(g2) : 0.0f, g1 = bf_hi(g2) > 0.0f ? bf_hi(g2) : 0.0f;
+        const uint32_t sq = f2bf_pair(g0 * g0, g1 * g1);
+        o[h] = f2bf_pair(bf_lo(sq) * bf_lo(u2), bf_hi(sq) * bf_hi(u2));
+      }
+    } else {
+      const uint32_t rw[4] = {res.x, res.y, res.z, res.w};
+#pragma unroll
+      for (int h = 0; h < 4; ++h) {
+        o[h] = f2bf_pair((float)e[0][2 * h] * f, (float)e[0][2 * h + 1] * f);
+        if (p.residual) o[h] = f2bf_pair(bf_lo(rw[h]) + bf_lo(o[h]), bf_hi(rw[h]) + bf_hi(o[h]));
+      }
+    }
+    *reinterpret_cast<uint4*>(p.out + at) = make_uint4(o[0], o[1], o[2], o[3]);
+  }
+}
+
 // ------------------------------------------------------------- planning --
 // Waves per standalone decode workgroup: 8 (two per SIMD) unless
 // BTL_DECODE_WAVES=4.  The fused kernel always runs 8.
@@ -1586,6 +1741,59 @@ static void launch_prefill_epi(bool prs, int rb, bool sk, dim3 grid, hipStream_t
   }
 }
 
+// Which k_gemm_rows instance a fused call with M > 32 runs, if any: 32 rows x
+// one tile (kRowsT), 32 rows x two tiles (kRowsA) or 128 rows x two tiles
+// (kRowsC) a workgroup.  Each takes about t0 + rounds * (a + b KS) us, rounds
+// the workgroups per CU (fitted on MI355X to KS = 8 .. 54, M = 40 .. 2048, within
+// 15 %); the quickest by that runs while 128-row workgroups fit the chip once
+// (twice for gate||up, whose alternative has no wide form) or 32-row ones three
+// times.  Beyond that the tile kernels, which read each operand once per tile
+// and not once per 64 columns, are level or ahead.  Measured, tile kernel ->
+// this (us): 2560 -> 2 x 6912 relu2 M = 64 / 128 / 256: 14.4 / 14.3 / 15.2 ->
+// 6.8 / 8.9 / 13.7, M = 512 (not taken) 21.6 / 24.3; 6912 -> 2560 M = 64 / 128 /
+// 256 / 512 / 768: 19.2 / 20.2 / 20.1 / 21.3 / 23.1 -> 5.2 / 6.7 / 10.4 / 14.4 /
+// 18.3, M = 1024 (not taken) 26.8 / 31.3; 2560 -> 3840 M = 128 / 256 / 512: 15.1 /
+// 10.9 / 11.9 -> 4.5 / 6.2 / 9.6; 640 -> 160 M = 40 .. 2048: 6.6 .. 4.9 -> 3.2 .. 3.7.
+enum RowsKind { kRowsNone, kRowsT, kRowsA, kRowsC };
+static RowsKind rows_plan(int64_t M, int64_t K, int64_t N, int epilogue) {
+  const int64_t Mb = mblocks(M), NT = N / 32, KS = ksb(K), cus = device_cus();
+  const bool relu2 = epilogue == BTL_EPI_RELU2_MUL;
+  if (M <= 32 || M > (1 << 15)) return kRowsNone;
+  auto rounds = [&](int64_t wgs) { return (wgs + cus - 1) / cus; };
+  const int64_t pairs = relu2 ? NT / 2 : (NT + 1) / 2;
+  const int64_t nt = rounds(NT * Mb), na = rounds(pairs * Mb), nc = rounds(pairs * ((Mb + 3) / 4));
+  if (nc > (relu2 ? 2 : 1) && na > 3) return kRowsNone;
+  const double tt = 2.2 + (double)nt * (0.65 + 0.045 * (double)KS);
+  const double ta = 2.4 + (double)na * (0.9 + 0.055 * (double)KS);
+  const double tc = 3.2 + (double)nc * (1.3 + 0.24 * (double)KS);
+  if (!relu2 && tt <= ta && tt <= tc) return kRowsT;
+  return ta <= tc ? kRowsA : kRowsC;
+}
+
+template <int RBW, int RH, int TPW, int D, int EPI>
+static void launch_rows(hipStream_t s, const GemmArgs& a) {
+  const int ngm = (a.Mb + RBW * RH - 1) / (RBW * RH);
+  const int ngn = EPI == EPI_RELU2 ? (a.NT / 2 + TPW / 2 - 1) / (TPW / 2) : (a.NT + TPW - 1) / TPW;
+  const int per = (ngm * ngn + kPfXcds - 1) / kPfXcds;
+  hipLaunchKernelGGL((k_gemm_rows<RBW, RH, TPW, D, EPI>), dim3((unsigned)(per * kPfXcds)), dim3(512), 0, s, a, ngm,
+                     ngn);
+}
+static int launch_gemm_rows(RowsKind kind, const GemmArgs& a, int epilogue, hipStream_t s) {
+  if (epilogue == BTL_EPI_RELU2_MUL) {
+    if (kind == kRowsA)
+      launch_rows<1, 1, 2, 1, EPI_RELU2>(s, a);
+    else
+      launch_rows<1, 4, 2, 1, EPI_RELU2>(s, a);
+  } else if (kind == kRowsT) {
+    launch_rows<1, 1, 1, 2, EPI_SCALE>(s, a);
+  } else if (kind == kRowsA) {
+    launch_rows<1, 1, 2, 1, EPI_SCALE>(s, a);
+  } else {
+    launch_rows<1, 4, 2, 1, EPI_SCALE>(s, a);
+  }
+  return check_launch("ternary gemm (few rows)");
+}
+
 static int launch_gemm(const GemmArgs& a, int epilogue, const GemmPlan& pl, hipStream_t s) {
   if (pl.prefill) {
     WidePlan w;
@@ -1780,7 +1988,9 @@ static int bitlinear_fused_impl(const uint16_t* x, int64_t M, int64_t K, int64_t
     clear_error();
   }
 
-  const GemmPlan pl = plan_gemm(M, K, N, epilogue, splitk);
+  GemmPlan pl = plan_gemm(M, K, N, epilogue, splitk);
+  const RowsKind rows = rows_plan(M, K, N, epilogue);
+  if (rows != kRowsNone) pl.splitk = 1;  // no partials, no counters
   // The prefill GEMM takes the row sums from the activation kernel, which
   // has them in registers anyway; the decode GEMM sums its own operand.
   int32_t* rowsum = pl.prefill ? (int32_t*)(ws + L.rowsum) : nullptr;
@@ -1789,6 +1999,7 @@ static int bitlinear_fused_impl(const uint16_t* x, int64_t M, int64_t K, int64_t
   if (rc) return rc;
   const GemmArgs g = gemm_args(xa, a_dq, rowsum, M, K, N, wdev, seg_scale, seg_end, nseg, epilogue, residual, out,
                                acc_out, ws + L.gemm_ws, pl);
+  if (rows != kRowsNone) return launch_gemm_rows(rows, g, epilogue, s);
   return launch_gemm(g, epilogue, pl, s);
 }
 
