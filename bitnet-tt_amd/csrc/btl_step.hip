@@ -2,6 +2,8 @@
 // model as one persistent launch on gfx950 (every layer's QKV, o_proj,
 // gate||up and down; src/bitnet_tt/inference/generator_batch32.py:713-761).
 //
+// A batch of one has a kernel of its own (k_decode_step_one, below).
+//
 // Roles.  One workgroup per CU, 512 threads.
 //   Row workgroups 0..31: one token row each.  A row workgroup keeps its row
 //     of the residual stream (hidden) in registers for the whole step and runs
@@ -733,10 +735,10 @@ __device__ __forceinline__ void wait_tile_piece(const StepArgs& p, __amdgpu_buff
 // v_mfma_i32_16x16x64_i8: a 32-lane and then a 16-lane swap of the words of
 // 32-k steps 2p and 2p + 1 give lane l column (l & 15) (word 2p) and column
 // 16 + (l & 15) (word 2p + 1), each with k-group l >> 4 of the 64-k step.
-template <int TPW, int NSW>
-__device__ __forceinline__ void regroup_half_weights(v4i (&w)[kStepWSlots]) {
+template <int N, int S>
+__device__ __forceinline__ void regroup_words(v4i (&w)[S]) {
 #pragma unroll
-  for (int s = 0; s < TPW * NSW; ++s)
+  for (int s = 0; s < N; ++s)
 #pragma unroll
     for (int pp = 0; pp < 2; ++pp) {
       const auto s32 = __builtin_amdgcn_permlane32_swap((uint32_t)w[s][2 * pp], (uint32_t)w[s][2 * pp + 1], false,
@@ -768,7 +770,7 @@ __device__ void step_gemm_op(const StepArgs& p, const StepOp* sops, int l, int g
   constexpr int NR = OpShape<J, A>::HALF ? 16 : 32;  // rows of the unit
   // A 16-row unit's weight words are regrouped for its MFMA before the flags
   // are awaited (they were loaded during the previous hand-off).
-  if constexpr (OpShape<J, A>::HALF) regroup_half_weights<TPW, NSW>(w);
+  if constexpr (OpShape<J, A>::HALF) regroup_words<TPW * NSW>(w);
   if (wv == kStepPollWave) wait_flags(p, l, J, 16 * h, NR, want, s_adq, ws);
   lds_barrier();  // the rows' flags are in (no wait for loads in flight)
   STEP_TRACE(l, 8 + 2 * J);
@@ -847,7 +849,7 @@ __device__ void step_gemm_op(const StepArgs& p, const StepOp* sops, int l, int g
       load();
       v4i wr[kStepWSlots];
       load_unit_weights<J, NSW, A>(p, sops, l, gi, wr);
-      regroup_half_weights<TPW, NSW>(wr);
+      regroup_words<TPW * NSW>(wr);
       (void)mfma(wr);
     }
 #pragma unroll
@@ -1218,6 +1220,319 @@ __global__ __launch_bounds__(512) void k_decode_step(StepArgs p) {
   if (threadIdx.x == 0) p.epoch[b] = E;
 }
 
+// ----------------------------------------------------------- one user ----
+// The step for a batch of one: one hand-off per BitLinear instead of two.
+// With one row every unit can afford the row work itself: it polls the previous
+// BitLinear's tagged output words (10 KB at K = 2560), runs the residual add,
+// RMSNorm, absmax and quantisation into its own LDS (the residual stream lives
+// in every workgroup's registers), and multiplies from there: no row
+// workgroup, operand tile, flags or sentinels, and one hop less per BitLinear.
+// Measured on MI355X, six layers of the 2B model, two hops -> one: the
+// BitLinears 118.5 -> 101.0 us; with the attention 147.3 -> 118.8 at position
+// 37, 151.7 -> 124.3 at 511, 172.7 -> 144.0 at 4000.  The same for two and four
+// rows was slower than two hops (121.9 -> 140.8, 124.2 -> 210.9): each row adds
+// 1 us of row work to every stage of every unit.  The polling is not what
+// bounds it: longer sleeps between polls are slower.
+//
+// Workgroup u is unit u of each BitLinear: column tile u (gate||up: gate tile u
+// and its up tile), all of K, the 8 waves splitting the superblocks; the last
+// workgroups, which have no unit, take an attention item each.  Every row of
+// v_mfma_i32_16x16x64_i8 gets the one row (all lanes of a k-group read the same
+// 16 bytes), so element 0 of lanes 0-15 is the result.  Weights and gains are
+// loaded one layer ahead, each right after the poll that follows its last use:
+// a load ahead of a poll would hold the poll back, and between two polls there
+// is the row work to hide it.
+//
+// The tagged words are reused by every layer.  Every reader of BitLinear j's
+// words of layer l has, before it produces any word of a later BitLinear of
+// its own, read them; and a unit writes j's words of layer l + 1 only with
+// inputs that depend on words of every unit of each BitLinear in between,
+// hence of every such reader: the workgroups that follow the residual stream
+// are the units of QKV and gate||up, o_proj's words are read by those and
+// QKV's by o_proj's units or the attention items.
+constexpr int kOneRed = 8192 / 4;                         // LDS ints: the quantised row, then partial sums
+constexpr int kOneStat = kOneRed + kStepWaves * 2 * 32;   // [8 waves][2 tiles][32]; then the waves' statistics
+static_assert(kOneStat + 16 <= kStepIdxInt, "LDS below the unit index words");
+
+template <int J>
+struct OneShape {
+  static constexpr int TPW = J == S_GU ? 2 : 1;
+};
+// This wave's weights of unit u of BitLinear J, and this thread's gains.
+template <int J, int NSW, int C>
+__device__ __forceinline__ void one_load(const StepArgs& p, const StepOp* sops, int l, int u,
+                                         v4i (&w)[OneShape<J>::TPW * NSW], uint4 (&g)[C]) {
+  if (l >= p.L || u >= op_n(p, J) / 32 / OneShape<J>::TPW) return;  // uniform
+  const int tid = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int KS = op_ks(p, J), nch = KS * 16;
+  const StepOp& op = sops[l * kStepOps + J];
+#pragma unroll
+  for (int i = 0; i < C; ++i) {
+    const v4i t = ldg128(op.gamma + 8 * min(tid + kActThreads * i, nch - 1));
+    g[i] = make_uint4((uint32_t)t.x, (uint32_t)t.y, (uint32_t)t.z, (uint32_t)t.w);
+  }
+  int wb, we;
+  wave_ks(0, KS, wv, wb, we);
+  if (wb >= we) return;  // wave-uniform: no superblock
+#pragma unroll
+  for (int t = 0; t < OneShape<J>::TPW; ++t) {
+    const int tile = unit_tile<J>(p, u, t);
+#pragma unroll
+    for (int i = 0; i < NSW; ++i)
+      w[t * NSW + i] = ldg128(op.wdev + (((int64_t)tile * KS + min(wb + i, we - 1)) * 64 + lane) * 4);
+  }
+}
+
+// RMSNorm, absmax and quantisation of the row (v: this thread's chunks) into
+// LDS, the arithmetic and order of publish_row; returns a/127.  Its barriers
+// do not wait for the weights in flight.
+template <int C>
+__device__ __forceinline__ float one_quant(const StepArgs& p, int K, float (&v)[C][8], const uint4 (&graw)[C],
+                                           int32_t* lds) {
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, nch = K >> 3;
+  float* s_sum = reinterpret_cast<float*>(lds + kOneStat);
+  uint32_t* s_max = reinterpret_cast<uint32_t*>(lds + kOneStat + 8);
+  float s = 0.0f;
+#pragma unroll
+  for (int i = 0; i < C; ++i)
+    if (tid + kActThreads * i < nch) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float sq = v[i][j] * v[i][j];
+        s = s + sq;
+      }
+    }
+  s = wave_xor_sum(s);
+  if (lane == 0) s_sum[wv] = s;
+  float g[C][8];
+  gains_to_floats<C>(graw, g);
+  lds_barrier();
+  const float var = sum8_fixed(s_sum) / (float)K;
+  row_apply_norm_f<C>(v, g, 1.0f / sqrtf(var + p.eps), nch, tid);
+  float amax = 0.0f;
+#pragma unroll
+  for (int i = 0; i < C; ++i)
+    if (tid + kActThreads * i < nch) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(v[i][j]));
+    }
+  uint32_t m = __float_as_uint(amax);
+  m = max(m, xor_partner_u<32>(m));
+  m = max(m, xor_partner_u<16>(m));
+  m = max(m, xor_partner_u<8>(m));
+  m = max(m, xor_partner_u<4>(m));
+  m = max(m, xor_partner_u<2>(m));
+  m = max(m, xor_partner_u<1>(m));
+  if (lane == 0) s_max[wv] = m;
+  lds_barrier();
+  m = s_max[0];
+#pragma unroll
+  for (int w = 1; w < kActWaves; ++w) m = max(m, s_max[w]);
+  const float am = __uint_as_float(m), a = am > 1e-5f ? am : 1e-5f;
+  const float scale = 127.0f / a;
+  int rs = 0;  // the units sum the operand bytes on the matrix pipe
+#pragma unroll
+  for (int i = 0; i < C; ++i) {
+    const int c = tid + kActThreads * i;
+    uint32_t lo, hi;
+    quant8(v[i], scale, lo, hi, rs);
+    if (c < nch) *reinterpret_cast<uint2*>(reinterpret_cast<uint8_t*>(lds) + 8 * c) = make_uint2(lo, hi);
+  }
+  lds_barrier();
+  return a / 127.0f;
+}
+
+// Unit u of BitLinear J of layer l from the row in LDS: MFMA, reduction over
+// the waves, epilogue (tagged words, and the caller's copy).  w: regrouped.
+template <int J, int NSW>
+__device__ __forceinline__ void one_gemm(const StepArgs& p, const StepOp* sops, int l, int u, uint32_t E,
+                                         const v4i (&w)[OneShape<J>::TPW * NSW], float ad, int32_t* lds) {
+  constexpr int TPW = OneShape<J>::TPW;
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int wb, we;
+  wave_ks(0, op_ks(p, J), wv, wb, we);
+  const StepOp& op = sops[l * kStepOps + J];
+  const int n = u * 32 + (tid & 31);
+  // segment scales: LDS reads, off the epilogue's path
+  const float sc0 = op_seg_scale(op, n);
+  const float sc1 = J == S_GU ? op_seg_scale(op, unit_tile<J>(p, u, 1) * 32) : 0.0f;
+  const uint8_t* row = reinterpret_cast<const uint8_t*>(lds) + (lane >> 4) * 16;
+  v4i acc[TPW][2], acc_rs = {0, 0, 0, 0};
+#pragma unroll
+  for (int t = 0; t < TPW; ++t) acc[t][0] = acc[t][1] = (v4i){0, 0, 0, 0};
+  const v4i ones = {0x01010101, 0x01010101, 0x01010101, 0x01010101};
+#pragma unroll
+  for (int i = 0; i < NSW; ++i)
+    if (wb + i < we)
+#pragma unroll
+      for (int pp = 0; pp < 2; ++pp) {
+        const v4i a = *reinterpret_cast<const v4i*>(row + (wb + i) * 128 + pp * 64);
+        acc_rs = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, ones, acc_rs, 0, 0, 0);
+#pragma unroll
+        for (int t = 0; t < TPW; ++t) {
+          acc[t][0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, unpack_b((uint32_t)w[t * NSW + i][2 * pp]), acc[t][0],
+                                                            0, 0, 0);
+          acc[t][1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, unpack_b((uint32_t)w[t * NSW + i][2 * pp + 1]),
+                                                            acc[t][1], 0, 0, 0);
+        }
+      }
+  int32_t* const red = lds + kOneRed;
+  if (lane < 16)
+#pragma unroll
+    for (int t = 0; t < TPW; ++t)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) red[(wv * TPW + t) * 32 + 16 * h + lane] = acc[t][h][0] - acc_rs[0];
+  lds_barrier();
+  if (tid < 32) {
+    int32_t sum[TPW];
+#pragma unroll
+    for (int t = 0; t < TPW; ++t) {
+      sum[t] = 0;
+#pragma unroll
+      for (int v2 = 0; v2 < kStepWaves; ++v2) sum[t] += red[(v2 * TPW + t) * 32 + tid];
+    }
+    uint32_t o = f2bf((float)sum[0] * (sc0 * ad));
+    if constexpr (J == S_GU) {
+      const float gg = bf2f((uint16_t)o);
+      const float uu = bf2f(f2bf((float)sum[1] * (sc1 * ad)));
+      const float gr = gg > 0.0f ? gg : 0.0f;
+      const float sq = bf2f(f2bf(gr * gr));
+      o = f2bf(sq * uu);
+    }
+    const uint32_t pair = o | (xor_partner_u<1>(o) << 16);  // two neighbouring columns (a DPP swap)
+    if ((tid & 1) == 0) {
+      st_coherent(out_of(p, l, J) + (n >> 1), ((uint64_t)step_tag(E, l, J) << 32) | pair);
+      if (J == S_QKV) *reinterpret_cast<uint32_t*>(p.qkv_out + n) = pair;
+      if (J == S_GU) *reinterpret_cast<uint32_t*>(p.ffn_h + n) = pair;
+    }
+  }
+}
+
+template <int CF, int NQ, int NDN, int ATT>
+__global__ __launch_bounds__(512) void k_decode_step_one(StepArgs p) {
+  // as k_decode_step: the op table above, and more than half of a CU's LDS
+  __shared__ __attribute__((aligned(16))) int32_t lds[24576];
+  constexpr int kTableInts = kStepMaxLayers * kStepOps * (int)sizeof(StepOp) / 4;
+  StepOp* sops = reinterpret_cast<StepOp*>(lds + (24576 - kTableInts));
+  const int tid = threadIdx.x, u = blockIdx.x;
+  {
+    const uint4* src = reinterpret_cast<const uint4*>(p.ops);
+    uint4* dst = reinterpret_cast<uint4*>(sops);
+    const int n16 = p.L * kStepOps * (int)sizeof(StepOp) / 16;
+    for (int i = tid; i < n16; i += blockDim.x) dst[i] = src[i];
+    if (tid == 0) lds[kStepIdxInt + 1] = 0;  // the attention body's opaque zero
+  }
+  __syncthreads();
+  const uint32_t E = p.epoch[u] + 1u;
+  WaitState ws{false, false};
+  if (ATT) {
+    const int ai = u - ((int)gridDim.x - p.Hkv * (ATT == 2 ? p.smax : 1));
+    if (ai >= 0) {  // an attention workgroup: no unit, so its caches travel from the layer's start
+      for (int l = 0; l < p.L; ++l) step_attention<ATT == 2>(p, l, ai, E, lds, ws);
+      if (tid == 0) p.epoch[u] = E;
+      return;
+    }
+  }
+  const int nh = p.H >> 3;
+  const bool uq = u < p.NQKV / 32, uo = u < p.H / 32, ug = u < p.F / 32;
+  const bool follows = uq || ug;  // holds the residual stream
+  v4i wq[NQ], wo[NQ], wg[2 * NQ], wd[NDN];
+  uint4 gq[1], go[1], gg[1], gd[CF];
+  one_load<S_QKV, NQ, 1>(p, sops, 0, u, wq, gq);
+  one_load<S_O, NQ, 1>(p, sops, 0, u, wo, go);
+  one_load<S_GU, NQ, 1>(p, sops, 0, u, wg, gg);
+  one_load<S_DN, NDN, CF>(p, sops, 0, u, wd, gd);
+  uint32_t hid[1][4];
+  {
+    uint4 raw = make_uint4(0u, 0u, 0u, 0u);
+    if (follows && tid < nh) raw = *reinterpret_cast<const uint4*>(p.hidden + 8 * tid);
+    hid[0][0] = raw.x;
+    hid[0][1] = raw.y;
+    hid[0][2] = raw.z;
+    hid[0][3] = raw.w;
+  }
+  // Weight words are regrouped ahead of the poll before their use (they landed
+  // a layer ago).
+  for (int l = 0; l < p.L; ++l) {
+    // ---- QKV: RMSNorm(h; input_layernorm), h = bf16(h + d) of the layer before
+    if (uq) regroup_words<NQ>(wq);
+    if (l > 0) {
+      if (follows) {
+        uint32_t pr[1][4];
+        wait_row_words<1>(p, out_of(p, l - 1, S_DN), p.H, step_tag(E, l - 1, S_DN), pr, ws);
+        residual_add(hid[0], pr[0], true);
+      }
+      one_load<S_DN, NDN, CF>(p, sops, l, u, wd, gd);
+    }
+    if (uq) {
+      float v[1][8];
+      pairs_to_floats<1>(hid, v);
+      const float ad = one_quant<1>(p, p.H, v, gq, lds);
+      one_gemm<S_QKV, NQ>(p, sops, l, u, E, wq, ad, lds);
+    }
+    // ---- O: RMSNorm(attn; attn_sub_norm)
+    if (uo) {
+      regroup_words<NQ>(wo);
+      uint32_t pr[1][4];
+      if (ATT) {
+        wait_row_words<1>(p, att_of(p), p.H, step_tag(E, l, 0), pr, ws);
+      } else {
+        // the attention output stand-in, once the user's QKV row, which
+        // attention would read, is in
+        uint4 raw = make_uint4(0u, 0u, 0u, 0u);
+        if (tid < nh) raw = *reinterpret_cast<const uint4*>(p.attn + 8 * tid);
+        wait_row_words<1>(p, out_of(p, l, S_QKV), p.NQKV, step_tag(E, l, S_QKV), pr, ws);
+        pr[0][0] = raw.x;
+        pr[0][1] = raw.y;
+        pr[0][2] = raw.z;
+        pr[0][3] = raw.w;
+      }
+      one_load<S_QKV, NQ, 1>(p, sops, l + 1, u, wq, gq);
+      float v[1][8];
+      pairs_to_floats<1>(pr, v);
+      const float ad = one_quant<1>(p, p.H, v, go, lds);
+      one_gemm<S_O, NQ>(p, sops, l, u, E, wo, ad, lds);
+    } else {
+      one_load<S_QKV, NQ, 1>(p, sops, l + 1, u, wq, gq);
+    }
+    // ---- GU: h = bf16(h + o); RMSNorm(h; post_attention_layernorm)
+    if (ug) regroup_words<2 * NQ>(wg);
+    if (follows) {
+      uint32_t pr[1][4];
+      wait_row_words<1>(p, out_of(p, l, S_O), p.H, step_tag(E, l, S_O), pr, ws);
+      residual_add(hid[0], pr[0], true);
+    }
+    one_load<S_O, NQ, 1>(p, sops, l + 1, u, wo, go);
+    if (ug) {
+      float v[1][8];
+      pairs_to_floats<1>(hid, v);
+      const float ad = one_quant<1>(p, p.H, v, gg, lds);
+      one_gemm<S_GU, NQ>(p, sops, l, u, E, wg, ad, lds);
+    }
+    // ---- DN: RMSNorm(relu(g)^2 * u; ffn_sub_norm)
+    if (uo) {
+      regroup_words<NDN>(wd);
+      uint32_t pr[CF][4];
+      wait_row_words<CF>(p, out_of(p, l, S_GU), p.F, step_tag(E, l, S_GU), pr, ws);
+      one_load<S_GU, NQ, 1>(p, sops, l + 1, u, wg, gg);
+      float v[CF][8];
+      pairs_to_floats<CF>(pr, v);
+      const float ad = one_quant<CF>(p, p.F, v, gd, lds);
+      one_gemm<S_DN, NDN>(p, sops, l, u, E, wd, ad, lds);
+    } else {
+      one_load<S_GU, NQ, 1>(p, sops, l + 1, u, wg, gg);
+    }
+  }
+  if (u == 0) {  // h = bf16(h + d) of the last layer
+    uint32_t pr[1][4];
+    wait_row_words<1>(p, out_of(p, p.L - 1, S_DN), p.H, step_tag(E, p.L - 1, S_DN), pr, ws);
+    residual_add(hid[0], pr[0], true);
+    if (tid < nh)
+      *reinterpret_cast<uint4*>(p.hidden + 8 * tid) = make_uint4(hid[0][0], hid[0][1], hid[0][2], hid[0][3]);
+  }
+  if (tid == 0) p.epoch[u] = E;
+}
+
 // ------------------------------------------------------- hand-off floor ----
 // The step's launch structure with no arithmetic, for measurement: per
 // BitLinear the row workgroups wait for every word of their row of the
@@ -1343,6 +1658,15 @@ static void (*step_kernel_fn(int64_t F, int att))(StepArgs) {
   if (cf == 2) return att == 2 ? k_decode_step<2, 3, 7, 2> : att ? k_decode_step<2, 3, 7, 1> : k_decode_step<2, 3, 7, 0>;
   return nullptr;
 }
+// The one-user kernel's instance, as above.
+static void (*step_one_fn(int64_t F, int att))(StepArgs) {
+  const int cf = act_cpt(F);
+  if (cf == 1)
+    return att == 2 ? k_decode_step_one<1, 3, 7, 2> : att ? k_decode_step_one<1, 3, 7, 1> : k_decode_step_one<1, 3, 7, 0>;
+  if (cf == 2)
+    return att == 2 ? k_decode_step_one<2, 3, 7, 2> : att ? k_decode_step_one<2, 3, 7, 1> : k_decode_step_one<2, 3, 7, 0>;
+  return nullptr;
+}
 static const void* step_kernel(int64_t F, bool floor, int att = 0) {
   const int cf = act_cpt(F);
   if (floor) return cf == 1 ? reinterpret_cast<const void*>(k_decode_step_floor<1>)
@@ -1401,7 +1725,12 @@ static StepArgs step_args(int64_t M, int64_t H, int64_t F, int64_t NQKV, int64_t
 }
 
 static int launch_step(const StepArgs& a, int64_t F, int att, const char* who, hipStream_t s) {
-  void (*k)(StepArgs) = step_kernel_fn(F, att);
+  // One user: the kernel whose units do the row work themselves, where the
+  // attention items leave every unit a workgroup of its own.
+  const int64_t units = std::max({a.NQKV / 32, a.H / 32, a.F / 32});
+  const int64_t items = att ? (int64_t)a.Hkv * a.smax : 0;
+  const bool one = a.M == 1 && units + items <= step_grid();
+  void (*k)(StepArgs) = one ? step_one_fn(F, att) : step_kernel_fn(F, att);
   if (!k) return set_error(BTL_ERR_SHAPE, "%s: no kernel instance for F=%lld", who, (long long)F);
   const int grid = step_grid();
   const int rc = check_coresident_launch(who, reinterpret_cast<const void*>(k), 512, grid, s);

@@ -395,3 +395,37 @@ def test_persistent_full_step_split_contexts(orc, batch, kv, S):
         step.step_persistent_full()
         step.check()
         _compare(_outputs(step), ref, f"split contexts, back {back}")
+
+
+# Batch 1, whose step has a kernel of its own: whole and split contexts, two
+# chunks of F per thread, and a shape whose 216 units and 64 attention items do
+# not fit 256 workgroups (the two-hop kernel).
+ONE_USER_FULL = [
+    (dict(num_layers=2, num_attention_heads=4, num_key_value_heads=1, hidden_size=512, intermediate_size=512), 256),
+    (dict(num_layers=3, num_attention_heads=16, num_key_value_heads=8, hidden_size=2048, intermediate_size=512), 1000),
+    (dict(num_layers=2, num_attention_heads=20, num_key_value_heads=5, hidden_size=2560, intermediate_size=6912), 4096),
+    (dict(num_layers=1, num_attention_heads=16, num_key_value_heads=8, hidden_size=2048, intermediate_size=6912), 4096),
+]
+
+
+@pytest.mark.parametrize("shape,S", ONE_USER_FULL)
+def test_one_user_full_step_matches_step_full(orc, shape, S):
+    """The one-launch step with attention at batch 1 against step_full, bit for
+    bit, at an early, a middle and the last position."""
+    from bitnet_tt.config import BitNetMiniConfig
+    from bitnet_tt.decode import BitLinearDecodeStep
+
+    print(f"one-user full step {shape} S={S}", flush=True)
+    step = BitLinearDecodeStep.random_init(BitNetMiniConfig(**shape), H.dev(), seed=83, batch=1).alloc_buffers(seed=84)
+    step.alloc_attention(max_seq_len=S)
+    for pos in (0, S // 2 + 3, S - 1):
+        step.pos.fill_(pos)
+        state = _full_state(step)
+        step.step_full()
+        step.check()
+        ref = _outputs(step)
+        for rep in range(3):
+            _restore(step, state)
+            step.step_persistent_full()
+            step.check()
+            _compare(_outputs(step), ref, f"one user, pos {pos}, rep {rep}")

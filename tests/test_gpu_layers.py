@@ -487,3 +487,48 @@ def test_models_taking_turns_keep_their_own_step_workspace(orc):
     del g, m, models
     gc.collect()
     assert not {k[3] for k in N._workspaces if len(k) == 4} & set(owners)
+
+
+# Batches of one run the kernel whose units do the row work themselves: more
+# QKV units than gate||up units and the reverse, one and two chunks of F per
+# thread, the 2B shape.
+ONE_USER_CONFIGS = [
+    dict(num_layers=3, num_attention_heads=2),
+    dict(num_layers=1, num_attention_heads=2, intermediate_size=128),
+    dict(num_layers=2, num_attention_heads=4, hidden_size=512, intermediate_size=4224),
+    dict(num_layers=2, num_attention_heads=20, num_key_value_heads=5, hidden_size=2560, intermediate_size=6912),
+]
+
+
+@pytest.mark.parametrize("shape", ONE_USER_CONFIGS)
+def test_one_user_step_matches_per_call(orc, shape):
+    """hidden, qkv and FFN rows of the one-launch step at batch 1 equal the
+    per-call chain's (pinned to the oracle elsewhere), over 50 graph replays
+    with the hand-off floor's launches on the same workspace between them."""
+    from bitnet_tt.config import BitNetMiniConfig
+    from bitnet_tt.decode import BitLinearDecodeStep
+
+    print(f"one-user step {shape}", flush=True)
+    step = BitLinearDecodeStep.random_init(BitNetMiniConfig(**shape), H.dev(), seed=81, batch=1).alloc_buffers(seed=82)
+    step.step_per_call()
+    ref = [t.clone() for t in (step.hidden, step.qkv_out, step.ffn_h)]
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(s):
+        step.step_persistent()
+    s.synchronize()
+    with torch.cuda.graph(g, stream=s):
+        step.step_persistent()
+    for rep in range(50):
+        step.reset_hidden()
+        torch.cuda.synchronize()
+        if rep % 10 == 3:
+            with torch.cuda.stream(s):
+                step.step_floor()
+        with torch.cuda.stream(s):
+            g.replay()
+        s.synchronize()
+        for got, want in zip((step.hidden, step.qkv_out, step.ffn_h), ref):
+            assert torch.equal(got, want), rep
+    step.check()
