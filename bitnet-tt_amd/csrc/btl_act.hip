@@ -1,4 +1,4 @@
-// Standalone activation prologue kernels: one or two waves per token row for
+// Standalone activation prologue kernels: one or four waves per token row for
 // the quantising prologue of batches of rows up to 8192 long, else one
 // workgroup of 512 threads per row running the row computation of
 // btl_act_row.h (RMSNorm, absmax int8 quantisation, blocked operand layout).  The fused decode kernel in
@@ -13,8 +13,8 @@ __global__ __launch_bounds__(kActThreads) void k_act_rows(ActArgs p) {
 }
 
 // The quantising prologue with one wave per row (four rows a workgroup) or
-// two (two rows): every row of a prefill batch in flight at once, with no
-// barrier (one wave) or a barrier between two waves (the 512-thread row above
+// four (one row): every row of a prefill batch in flight at once, with no
+// barrier (one wave) or barriers between four waves (the 512-thread row above
 // spends most of its time in two block reductions over eight waves and runs a
 // few hundred rows at a time).  The wave plays the eight waves of
 // act_row in turn: lane l holds the chunks of threads l, l + 64, ..., l + 448
@@ -24,8 +24,8 @@ __global__ __launch_bounds__(kActThreads) void k_act_rows(ActArgs p) {
 // and the row sum do not depend on the order.  Rows past M and columns past K
 // are written as zeros, as act_row writes them.
 constexpr int kActRowWaves = 4;  // waves a workgroup
-// WPR waves per row (1 or 2): wave h of a row takes the virtual waves
-// h * 8 / WPR .. and the two meet in LDS for the three row statistics.
+// WPR waves per row (1 or 4): wave h of a row takes the virtual waves
+// h * 8 / WPR .. and they meet in LDS for the three row statistics.
 template <bool NORM, int CPT, int WPR>
 __global__ __launch_bounds__(64 * kActRowWaves) void k_act_rows_wave(ActArgs p) {
   constexpr int NV = kActWaves;  // the 512-thread row's waves
@@ -52,7 +52,7 @@ __global__ __launch_bounds__(64 * kActRowWaves) void k_act_rows_wave(ActArgs p) 
       p.a_dq[m] = 0.0f;
       if (p.rowsum) p.rowsum[m] = 0;
     }
-    if (WPR == 1) return;  // with two waves a row it still takes part in the barriers
+    if (WPR == 1) return;  // with several waves a row it still takes part in the barriers
   }
   const uint16_t* xr = p.x + (int64_t)m * p.ldx;
   // chunk of (virtual wave w = h * NL + l, i): c = 64 w + lane + 512 i
@@ -139,10 +139,11 @@ __global__ __launch_bounds__(64 * kActRowWaves) void k_act_rows_wave(ActArgs p) 
   u = max(u, xor_partner_u<4>(u));
   u = max(u, xor_partner_u<2>(u));
   u = max(u, xor_partner_u<1>(u));
-  if constexpr (WPR == 2) {
+  if constexpr (WPR > 1) {
     if (lane == 0) s_mx[r][h] = u;
     __syncthreads();
-    u = max(s_mx[r][0], s_mx[r][1]);
+#pragma unroll
+    for (int w = 0; w < WPR; ++w) u = max(u, s_mx[r][w]);
   }
   const float amx = __uint_as_float(u);
   const float a = amx > p.act_eps ? amx : p.act_eps;
@@ -175,36 +176,34 @@ __global__ __launch_bounds__(64 * kActRowWaves) void k_act_rows_wave(ActArgs p) 
   if (!p.rowsum) return;
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) rs += __shfl_xor(rs, off, 64);
-  if constexpr (WPR == 2) {
+  if constexpr (WPR > 1) {
     if (lane == 0) s_rsum[r][h] = rs;
     __syncthreads();
-    rs = s_rsum[r][0] + s_rsum[r][1];
+    rs = 0;
+#pragma unroll
+    for (int w = 0; w < WPR; ++w) rs += s_rsum[r][w];
   }
   if (lane == 0 && h == 0 && !pad) p.rowsum[m] = rs;
 }
 
 template <bool NORM, bool QUANT>
 static void launch_rows(unsigned rows, hipStream_t s, const ActArgs& p) {
-  // rows is a multiple of 32 (whole row blocks) when quantising.  One wave
-  // per row from 1024 rows, two from 256, the 512-thread row below that
-  // (measured on MI355X, graph-timed: M = 2048, K = 2560 / 6912: 512-thread
-  // rows 10.6 / 17.9 us in a BitLinear sequence, one wave 9.5 / 14.3 us;
-  // M = 512: 512-thread rows 5.05 / 7.26 us, two waves 4.5 / 6.1 us, one wave
-  // 6.0 / 9.2 us; M = 100: 512-thread rows 3.6 us, two waves 4.3 us).
-  if (QUANT && act_cpt(p.K) <= 2 && rows >= 1024) {
-    const dim3 grid(rows / kActRowWaves), block(64 * kActRowWaves);
-    if (act_cpt(p.K) == 1)
-      hipLaunchKernelGGL((k_act_rows_wave<NORM, 1, 1>), grid, block, 0, s, p);
-    else
-      hipLaunchKernelGGL((k_act_rows_wave<NORM, 2, 1>), grid, block, 0, s, p);
-    return;
-  }
+  // rows is a multiple of 32 (whole row blocks) when quantising.  From 256 rows
+  // four waves a row; one wave from 1536 rows where it can skip blocks of the
+  // row past K (K <= 2560: five of eight in use); the 512-thread row below 256.
+  // Measured on MI355X, graph-timed, one / two / four waves a row (us):
+  // K = 2560, M = 256 / 511 / 1024 / 2048: - / 4.37 / 3.72, - / 4.52 / 4.14, 5.51 /
+  // 5.25 / 5.42, 7.97 / 8.79 / 8.55; K = 6912: - / 5.66 / 4.44, - / 6.33 / 5.75,
+  // 10.5 / 9.7 / 9.0, 15.2 / 14.2 / 13.5; K = 4096, M = 2048: 11.1 / 9.8 / 9.8; M = 100
+  // in 512-thread rows 3.65 (K = 2560), 4.4 (6912).
   if (QUANT && act_cpt(p.K) <= 2 && rows >= 256) {
-    const dim3 grid(rows / (kActRowWaves / 2)), block(64 * kActRowWaves);
-    if (act_cpt(p.K) == 1)
-      hipLaunchKernelGGL((k_act_rows_wave<NORM, 1, 2>), grid, block, 0, s, p);
+    const dim3 block(64 * kActRowWaves);
+    if (p.K <= 2560 && rows >= 1536)
+      hipLaunchKernelGGL((k_act_rows_wave<NORM, 1, 1>), dim3(rows / kActRowWaves), block, 0, s, p);
+    else if (act_cpt(p.K) == 1)
+      hipLaunchKernelGGL((k_act_rows_wave<NORM, 1, kActRowWaves>), dim3(rows), block, 0, s, p);
     else
-      hipLaunchKernelGGL((k_act_rows_wave<NORM, 2, 2>), grid, block, 0, s, p);
+      hipLaunchKernelGGL((k_act_rows_wave<NORM, 2, kActRowWaves>), dim3(rows), block, 0, s, p);
     return;
   }
   switch (act_cpt(p.K)) {

@@ -33,10 +33,9 @@ def run_quant(m, k, xb, gb=None, eps=1e-5):
                 scale=scale.cpu().numpy(), xq=xq.cpu().numpy(), y=H.bits_of(y))
 
 
-# For K <= 8192 the prologue runs two waves per row from 256 rows and one wave
-# per row from 1024: (300, 2560) and (500, 6912) take the first kernel,
-# (1000, 2560) and (1100, 6912) the second, with padding rows in the last row
-# block.
+# For K <= 8192 the prologue runs four waves per row from 256 rows ((300, 2560),
+# (500, 6912), (1000, 2560) and (1100, 6912), with padding rows in the last row
+# block); test_quant_absmax_wave_kernels has the one-wave rows and the edges.
 @pytest.mark.parametrize("m,k", [(1, 32), (5, 256), (32, 2560), (33, 2560), (70, 640), (32, 6912), (3, 16384),
                                  (300, 2560), (500, 6912), (1000, 2560), (1100, 6912)])
 @pytest.mark.parametrize("norm", [False, True])
@@ -58,6 +57,23 @@ def test_quant_absmax_bit_exact(orc, m, k, norm):
     # padding rows and columns are zero, as are their scales
     assert not full[m:].any() and not full[:, k:].any()
     assert not r["a_dq"][m:].any() and not r["rowsum"][m:].any()
+
+
+@pytest.mark.parametrize("m,k", [(225, 2560), (256, 64), (257, 8192), (400, 4128), (1504, 2560), (1505, 2560),
+                                 (1601, 2528), (1550, 32), (1540, 2592)])
+def test_quant_absmax_wave_kernels(orc, m, k):
+    """Edges of the wave-per-row kernels (M = 225 is the first row count in 256
+    padded rows, 1505 the first in 1536; K = 2560 the last one-wave width, 4096
+    and 8192 the last of one and two chunks a thread), norm on, against the
+    oracle: codes, scales and row sums to the bit."""
+    print(f"quant wave kernels m={m} k={k}", flush=True)
+    xb = H.activations(orc, m, k, seed=m * 7 + k)
+    gb = H.gamma(orc, k, seed=k + 1)
+    r = run_quant(m, k, xb, gb)
+    q, scale, a_dq, rowsum = orc.act_quant_absmax(orc.bf16_to_f32(orc.rmsnorm_bf16(xb, gb, 1e-5, order=1)))
+    assert np.array_equal(r["xq"], q) and np.array_equal(r["rowsum"][:m], rowsum)
+    assert np.array_equal(r["a_dq"][:m], a_dq) and np.array_equal(r["scale"], scale.reshape(-1))
+    assert np.array_equal(r["xa"], H.rowmajor_to_xa(q))
 
 
 def test_quant_special_rows(orc):
