@@ -16,8 +16,9 @@ epilogues.  Two launch structures compute the same bits:
 * ``step_persistent``: the whole step's BitLinears as one ``btl_decode_step``
   launch (one workgroup per CU; 32 row workgroups run the elementwise stages
   of the token rows, the others one GEMM unit of each BitLinear, with weights
-  loaded one BitLinear ahead).  The fastest on MI355X (0.70 ms for the 2B
-  model's 30 layers); it needs the attention width equal to hidden and the
+  loaded one BitLinear ahead; a batch of one has a kernel with one hand-off
+  per BitLinear).  The fastest on MI355X (0.63 ms for the 2B model's 30
+  layers); it needs the attention width equal to hidden and the
   shape limits of include/btl.h.
 * ``step_per_call`` (the default ``step``, which takes any shape the fused
   op takes): one ``btl_bitlinear_fused`` launch per BitLinear (120 per
