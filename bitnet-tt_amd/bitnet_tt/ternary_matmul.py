@@ -142,7 +142,16 @@ def ternary_matmul(
 
 
 # The library reads these arrays during the call and never writes them.
-_segments = functools.lru_cache(maxsize=4096)(N.segments_arrays)
+_cached_segments = functools.lru_cache(maxsize=4096)(N.segments_arrays)
+
+
+def _segments(scales, ends):
+    """segments_arrays of a weight's segments, kept by their values: a scale
+    may be any object that converts to a float (a tensor or array may change
+    in place between calls).  Zeros are not kept: 0.0 and -0.0 are equal keys."""
+    scales = tuple(map(float, scales))
+    ends = tuple(map(int, ends))
+    return N.segments_arrays(scales, ends) if 0.0 in scales else _cached_segments(scales, ends)
 
 
 @functools.lru_cache(maxsize=4096)
@@ -218,7 +227,7 @@ def ternary_matmul_into(
         gamma = norm_weight.data_ptr()
         eps = float(norm_epsilon)
     if weight_scale is None:
-        sc, en, nseg = _segments(tuple(w.segment_scales), tuple(w.segment_ends))
+        sc, en, nseg = _segments(w.segment_scales, w.segment_ends)
     elif isinstance(weight_scale, (int, float)):
         sc, en, nseg = N.segments_arrays((float(weight_scale),), (Nf,))
     else:

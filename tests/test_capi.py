@@ -196,6 +196,24 @@ def test_python_errors_are_loud(L):
         N.check(2, "probe")
 
 
+def test_segment_arrays_follow_the_scales_values():
+    """The epilogue's scale arrays of a call hold the segment scales as they
+    are at the call: a tensor changed in place, a 0-d array (no hash), and
+    0.0 after -0.0 (equal keys) are read anew."""
+    torch = pytest.importorskip("torch")
+    from bitnet_tt.ternary_matmul import _segments
+
+    t = torch.tensor(0.5)
+    assert list(_segments((t,), (64,))[0]) == [0.5]
+    t.fill_(2.0)
+    assert list(_segments((t,), (64,))[0]) == [2.0]
+    sc, en, n = _segments([np.array(0.25), np.float32(4.0)], [np.int64(32), 64])
+    assert list(sc) == [0.25, 4.0] and list(en) == [32, 64] and n == 2
+    for z in (-0.0, 0.0, -0.0):
+        assert np.signbit(list(_segments((z,), (64,))[0])[0]) == np.signbit(z)
+    assert _segments((0.5,), (64,))[0] is _segments((0.5,), (64,))[0]
+
+
 def test_decode_step_sizes_and_argument_checks(L):
     # one hand-off region reused by every layer: the workspace does not grow with L
     ws1 = L.btl_decode_step_workspace_bytes(32, 2560, 6912, 3840, 1)
