@@ -237,6 +237,7 @@ def ternary_matmul_into(
         sc, en, nseg = N.segments_arrays(scales, tuple(w.segment_ends))
     index = x.device.index
     stream = N.raw_stream(index)
+    splitk = int(splitk)
     nbytes, off = _fused_bytes(index, M, K, Nf, epi, splitk)
     ws, ws_bytes, _ = N.workspace_ptr(index, nbytes, "bitlinear", off, stream)
     rc = N.lib().btl_bitlinear_fused(x.data_ptr(), M, K, K, gamma, eps, w.data.data_ptr(), Nf, sc, en, nseg, epi, res,

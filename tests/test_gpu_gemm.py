@@ -586,6 +586,19 @@ def test_check_after_call_raises_at_the_call(orc):
     assert np.array_equal(H.bits_of(lin(H.to_dev_bf16(xb))), ref["out"])
 
 
+@pytest.mark.parametrize("splitk", [np.int64(2), 2.0, True])
+def test_splitk_takes_any_number(orc, splitk):
+    """splitk may be any value that int() takes."""
+    from bitnet_tt.ternary_matmul import PackedTernaryWeight, ternary_matmul
+
+    m, k, n = 32, 512, 256
+    xb = H.activations(orc, m, k, seed=31)
+    w = H.ternary(k, n, seed=32)
+    pw = PackedTernaryWeight(device_weight(orc, w), k, n, (0.02,), (n,))
+    out = ternary_matmul(H.to_dev_bf16(xb), pw, splitk=splitk)
+    assert np.array_equal(H.bits_of(out), orc.bitlinear(xb, w, [0.02])["out"])
+
+
 def _hip():
     import ctypes
 
