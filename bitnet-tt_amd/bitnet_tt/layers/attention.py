@@ -92,16 +92,20 @@ class QKVProjection:
 
 
 @functools.lru_cache(maxsize=4096)
-def _attention_bytes(index: int, b: int, h: int, hkv: int, s: int) -> tuple[int, int]:
-    """(workspace bytes, error word offset) of an attention call on device ``index``."""
+def _attention_bytes(index: int, b: int, h: int, hkv: int, s: int) -> tuple[int, int, int]:
+    """(workspace bytes, error word offset, split scratch bytes) of an attention
+    call on device ``index``."""
     L = N.lib()
     return (int(L.btl_decode_attention_workspace_bytes(b, h, hkv, s)),
-            int(L.btl_decode_attention_error_offset(b, hkv)))
+            int(L.btl_decode_attention_error_offset(b, hkv)),
+            int(L.btl_decode_attention_split_bytes(b, hkv, s)))
 
 
 class KVCache:
     """Pre-allocated per-layer cache (attention.py KVCache): key_cache and
-    value_cache [batch, kv_heads, max_seq_len, head_dim] bf16."""
+    value_cache [batch, kv_heads, max_seq_len, head_dim] bf16.  ``split`` is
+    the scratch of calls whose contexts are split over several workgroups; it
+    is the cache's own, since calls on one cache are ordered."""
 
     def __init__(self, batch: int, num_kv_heads: int, max_seq_len: int, head_dim: int, device) -> None:
         import torch
@@ -109,6 +113,11 @@ class KVCache:
         shape = (batch, num_kv_heads, max_seq_len, head_dim)
         self.key_cache = torch.zeros(shape, dtype=torch.bfloat16, device=device)
         self.value_cache = torch.zeros(shape, dtype=torch.bfloat16, device=device)
+        self.split = None
+        if self.key_cache.is_cuda:
+            nbytes = int(N.lib().btl_decode_attention_split_bytes(batch, num_kv_heads, max_seq_len))
+            if nbytes:
+                self.split = torch.zeros(nbytes, dtype=torch.uint8, device=device)
         self.seq_len_cached = 0
 
 
@@ -151,7 +160,10 @@ class DecodeAttention:
     def __call__(self, qkv, kv_cache: KVCache, pos, out=None):
         """qkv bf16 [B, (H + 2 Hkv) D]; pos int32 [B] on the device (each user's
         new position; a device tensor so a captured graph can advance it);
-        returns bf16 [B, H D] (written into ``out`` when given)."""
+        returns bf16 [B, H D] (written into ``out`` when given).  Calls on one
+        cache, eager or replayed, must be ordered: each writes the cache's rows
+        and, where contexts are split over workgroups, its scratch.  A cache
+        object without a scratch of this shape gets whole contexts."""
         import torch
 
         B = qkv.shape[0]
@@ -168,14 +180,19 @@ class DecodeAttention:
             out = torch.empty((B, H * D), dtype=torch.bfloat16, device=qkv.device)
         index = qkv.device.index
         stream = N.raw_stream(index)
-        nbytes, off = _attention_bytes(index, B, H, Hkv, S)
+        nbytes, off, split_bytes = _attention_bytes(index, B, H, Hkv, S)
         if torch.cuda.is_current_stream_capturing() and not N.has_workspace(qkv.device, nbytes, "attention"):
             raise RuntimeError("run one eager attention call on this stream before capturing it in a graph")
         ws, ws_bytes, _ = N.workspace_ptr(index, nbytes, "attention", off, stream)
-        rc = N.lib().btl_decode_attention(
+        split = None
+        if split_bytes:
+            t = getattr(kv_cache, "split", None)
+            if t is not None and t.numel() >= split_bytes and t.device.index == index:
+                split = t.data_ptr()
+        rc = N.lib().btl_decode_attention_split(
             qkv.data_ptr(), B, H, Hkv, D, S, pos.data_ptr(), self.rope_cos.data_ptr(), self.rope_sin.data_ptr(),
             int(self.use_fused_rope), float(self.scale), kv_cache.key_cache.data_ptr(),
-            kv_cache.value_cache.data_ptr(), out.data_ptr(), ws, ws_bytes, stream)
+            kv_cache.value_cache.data_ptr(), out.data_ptr(), ws, ws_bytes, split, split_bytes, stream)
         if rc != N.BTL_OK:
             N.check(rc, "btl_decode_attention")
         return out

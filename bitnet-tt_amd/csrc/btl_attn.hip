@@ -9,14 +9,16 @@
 // caches [B, Hkv, S, D] bf16 (the reference's KV-cache shape); output
 // [B, H D] bf16 (heads concatenated, o_proj's input).  D = 128.
 //
-// One workgroup of 8 waves per (user, key-value head), or, where the pairs
-// leave most of the chip idle, one per split of a pair's context
-// (btl_attn_body.h): each split publishes its partial with coherent stores and
-// counts itself, and the last of a pair to arrive merges them in split order.
-// Nothing waits on another workgroup.  (At the 2B shape's 160 pairs and 512
-// positions the store-acknowledge-count-reload chain costs more than the
-// extra CUs gain: one split.)
+// One workgroup of 8 waves per (user, key-value head), or, where the caller
+// gives a scratch for it and the pairs leave most of the chip idle, one per
+// split of a pair's context (btl_attn_body.h): each split publishes its partial
+// with coherent stores and counts itself, and the last of a pair to arrive
+// merges them in split order.  Nothing waits on another workgroup.  (At the 2B
+// shape's 160 pairs and 512 positions the store-acknowledge-count-reload chain
+// costs more than the extra CUs gain: one split.)
 #include <hip/hip_runtime.h>
+
+#include <atomic>
 
 #include "btl.h"
 #include "btl_attn_body.h"
@@ -39,13 +41,19 @@ struct AttnArgs {
   float scale;
   int adjacent;            // 1: RoPE pairs (2i, 2i+1); 0: (i, i + D/2)
   int smax;                // workgroups per (user, key-value head)
-  uint32_t* count;         // [pairs] splits arrived (zero between calls)
+  // smax > 1.  A pair's arrival word is a call's number plus the splits that
+  // have arrived, which is zero between calls.  Every split raises the word to
+  // its own call's number before it arrives, so that a count left over from two
+  // calls that ran at once on one scratch does not outlive them.
+  uint64_t* arrive;        // [pairs]
+  uint64_t call;           // a multiple of kAttnCallStep, larger in each later call
   float* part;             // [pairs][smax][kAtPartFloats]
 };
+constexpr uint64_t kAttnCallStep = 16;  // > kAtMaxSplits
+static_assert(kAtMaxSplits < (int)kAttnCallStep, "arrivals fit below the call's number");
 
-// Workspace: the error word, then (smax > 1) the arrival counters and partials.
-constexpr int64_t kAttnCount = 256;
-constexpr int64_t kAttnPart = kAttnCount + kAtSplitItems * 4;
+constexpr int64_t kAttnWorkspace = 256;                // the error word
+constexpr int64_t kAttnPart = kAtSplitItems * 8;       // split scratch: the arrival words, then the partials
 static_assert(kAttnPart % 16 == 0, "partials aligned");
 
 // Publishes this split's partial; true in the workgroup that arrived last,
@@ -65,10 +73,14 @@ __device__ bool attn_gather(const AttnArgs& p, const AttnPair& a, int pair, int 
   }
   wait_memory();
   __syncthreads();  // the whole partial is out before the arrival is counted
-  if (tid == 0) *s_last = atomicAdd(p.count + pair, 1u) == (unsigned)(n - 1);
+  if (tid == 0) {
+    const uint64_t w = atomicAdd(reinterpret_cast<unsigned long long*>(p.arrive + pair), 1ull);
+    const uint64_t arrived = w % kAttnCallStep;
+    *s_last = arrived == (uint64_t)(n - 1);
+    if (*s_last) st_coherent(p.arrive + pair, w - arrived);  // left clean for the next call
+  }
   __syncthreads();
   if (!*s_last) return false;
-  if (tid == 0) st_coherent(p.count + pair, 0u);  // left clean for the next call
   const int gc = min(g, a.G - 1);
 #pragma unroll
   for (int i = 0; i < kAtMaxSplits; ++i)
@@ -124,8 +136,10 @@ __global__ __launch_bounds__(64 * kAtWaves, 1) void k_decode_attention(AttnArgs 
   __syncthreads();
   BTL_TRACE_AT(2);
   AttnPartial part;
-  uint16_t o = att_body(a, s, r, part, true);
   const int n = SPLIT ? a.splits() : 1;
+  // long before this split's own arrival, which waits for it
+  if (SPLIT && n > 1 && tid == 0) atomicMax(reinterpret_cast<unsigned long long*>(p.arrive + pair), p.call);
+  uint16_t o = att_body(a, s, r, part, true);
   if (SPLIT && n > 1) {
     float Ms[kAtMaxSplits], Ls[kAtMaxSplits], Os[kAtMaxSplits];
     if (!attn_gather(p, a, pair, n, part, &s_last, Ms, Ls, Os)) return;
@@ -145,9 +159,13 @@ extern "C" {
 
 int64_t btl_decode_attention_workspace_bytes(int64_t B, int64_t H, int64_t Hkv, int64_t S) {
   if (B <= 0 || Hkv <= 0 || H <= 0 || H % Hkv || H / Hkv > kAtMaxG || S <= 0) return 0;
-  // the error word; the counters and partials of the splits, where a call of
-  // this shape has any (at most kAtSplitItems, on any device)
-  if (S <= kAtWaves * kAtPosWave || 2 * B * Hkv > kAtSplitItems) return kAttnCount;
+  return kAttnWorkspace;
+}
+
+int64_t btl_decode_attention_split_bytes(int64_t B, int64_t Hkv, int64_t S) {
+  if (B <= 0 || Hkv <= 0 || S <= 0) return 0;
+  // at most kAtSplitItems splits, on any device
+  if (att_max_splits(B * Hkv, S, kAtSplitItems + 32) == 1) return 0;
   return kAttnPart + (int64_t)kAtSplitItems * kAtPartFloats * 4;
 }
 
@@ -157,24 +175,29 @@ int64_t btl_decode_attention_error_offset(int64_t B, int64_t Hkv) {
   return 0;
 }
 
-int btl_decode_attention(const uint16_t* qkv, int64_t B, int64_t H, int64_t Hkv, int64_t D, int64_t S,
-                         const int32_t* pos, const float* rope_cos, const float* rope_sin, int rope_adjacent,
-                         float scale, uint16_t* k_cache, uint16_t* v_cache, uint16_t* out, void* workspace,
-                         size_t workspace_bytes, btl_stream_t stream) {
+static int decode_attention(const char* who, const uint16_t* qkv, int64_t B, int64_t H, int64_t Hkv, int64_t D,
+                            int64_t S, const int32_t* pos, const float* rope_cos, const float* rope_sin,
+                            int rope_adjacent, float scale, uint16_t* k_cache, uint16_t* v_cache, uint16_t* out,
+                            void* workspace, size_t workspace_bytes, void* split, size_t split_bytes,
+                            btl_stream_t stream) {
   clear_error();
-  if (D != kAtD) return set_error(BTL_ERR_SHAPE, "btl_decode_attention: head dim %lld (128 supported)", (long long)D);
+  if (D != kAtD) return set_error(BTL_ERR_SHAPE, "%s: head dim %lld (128 supported)", who, (long long)D);
   if (B <= 0 || B > 4096 || Hkv <= 0 || H <= 0 || H % Hkv || H / Hkv > kAtMaxG || S <= 0 || S > (1 << 20))
-    return set_error(BTL_ERR_SHAPE, "btl_decode_attention: B=%lld H=%lld Hkv=%lld S=%lld (H/Hkv <= %d)",
-                     (long long)B, (long long)H, (long long)Hkv, (long long)S, kAtMaxG);
+    return set_error(BTL_ERR_SHAPE, "%s: B=%lld H=%lld Hkv=%lld S=%lld (H/Hkv <= %d)", who, (long long)B,
+                     (long long)H, (long long)Hkv, (long long)S, kAtMaxG);
   if (!qkv || !pos || !rope_cos || !rope_sin || !k_cache || !v_cache || !out || !workspace)
-    return set_error(BTL_ERR_NULL, "btl_decode_attention: NULL pointer");
+    return set_error(BTL_ERR_NULL, "%s: NULL pointer", who);
   if (!aligned(qkv, 16) || !aligned(k_cache, 16) || !aligned(v_cache, 16) || !aligned(out, 16) ||
-      !aligned(workspace, 256) || !aligned(pos, 4) || !aligned(rope_cos, 4) || !aligned(rope_sin, 4))
-    return set_error(BTL_ERR_ALIGN, "btl_decode_attention: misaligned buffer");
-  const int64_t need = btl_decode_attention_workspace_bytes(B, H, Hkv, S);
-  if ((int64_t)workspace_bytes < need)
-    return set_error(BTL_ERR_WORKSPACE, "btl_decode_attention: workspace %zu < %lld bytes", workspace_bytes,
-                     (long long)need);
+      !aligned(workspace, 256) || !aligned(pos, 4) || !aligned(rope_cos, 4) || !aligned(rope_sin, 4) ||
+      !aligned(split, 16))
+    return set_error(BTL_ERR_ALIGN, "%s: misaligned buffer", who);
+  if ((int64_t)workspace_bytes < kAttnWorkspace)
+    return set_error(BTL_ERR_WORKSPACE, "%s: workspace %zu < %lld bytes", who, workspace_bytes,
+                     (long long)kAttnWorkspace);
+  if (split && (int64_t)split_bytes < btl_decode_attention_split_bytes(B, Hkv, S))
+    return set_error(BTL_ERR_WORKSPACE, "%s: split scratch %zu < %lld bytes", who, split_bytes,
+                     (long long)btl_decode_attention_split_bytes(B, Hkv, S));
+  static std::atomic<uint64_t> calls{0};
   AttnArgs a;
   a.qkv = qkv;
   a.ldq = (int)((H + 2 * Hkv) * D);
@@ -192,15 +215,37 @@ int btl_decode_attention(const uint16_t* qkv, int64_t B, int64_t H, int64_t Hkv,
   a.scale = scale;
   a.adjacent = rope_adjacent ? 1 : 0;
   a.error = reinterpret_cast<int32_t*>(workspace);
-  a.smax = att_max_splits(B * Hkv, S, device_cus());
-  a.count = reinterpret_cast<uint32_t*>(static_cast<char*>(workspace) + kAttnCount);
-  a.part = reinterpret_cast<float*>(static_cast<char*>(workspace) + kAttnPart);
+  a.smax = split ? att_max_splits(B * Hkv, S, device_cus()) : 1;
+  a.arrive = nullptr;
+  a.call = 0;
+  a.part = nullptr;
+  if (a.smax > 1) {
+    a.arrive = reinterpret_cast<uint64_t*>(split);
+    a.call = kAttnCallStep * (calls.fetch_add(1, std::memory_order_relaxed) + 1);
+    a.part = reinterpret_cast<float*>(static_cast<char*>(split) + kAttnPart);
+  }
   const dim3 grid((unsigned)(B * Hkv * a.smax));
   if (a.smax > 1)
     hipLaunchKernelGGL(k_decode_attention<true>, grid, dim3(64 * kAtWaves), 0, (hipStream_t)stream, a);
   else
     hipLaunchKernelGGL(k_decode_attention<false>, grid, dim3(64 * kAtWaves), 0, (hipStream_t)stream, a);
   return check_launch("decode attention");
+}
+
+int btl_decode_attention(const uint16_t* qkv, int64_t B, int64_t H, int64_t Hkv, int64_t D, int64_t S,
+                         const int32_t* pos, const float* rope_cos, const float* rope_sin, int rope_adjacent,
+                         float scale, uint16_t* k_cache, uint16_t* v_cache, uint16_t* out, void* workspace,
+                         size_t workspace_bytes, btl_stream_t stream) {
+  return decode_attention("btl_decode_attention", qkv, B, H, Hkv, D, S, pos, rope_cos, rope_sin, rope_adjacent, scale,
+                          k_cache, v_cache, out, workspace, workspace_bytes, nullptr, 0, stream);
+}
+
+int btl_decode_attention_split(const uint16_t* qkv, int64_t B, int64_t H, int64_t Hkv, int64_t D, int64_t S,
+                               const int32_t* pos, const float* rope_cos, const float* rope_sin, int rope_adjacent,
+                               float scale, uint16_t* k_cache, uint16_t* v_cache, uint16_t* out, void* workspace,
+                               size_t workspace_bytes, void* split, size_t split_bytes, btl_stream_t stream) {
+  return decode_attention("btl_decode_attention_split", qkv, B, H, Hkv, D, S, pos, rope_cos, rope_sin, rope_adjacent,
+                          scale, k_cache, v_cache, out, workspace, workspace_bytes, split, split_bytes, stream);
 }
 
 }  // extern "C"

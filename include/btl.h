@@ -381,16 +381,26 @@ int btl_lm_head(const uint16_t* xn, int64_t M, int64_t K, int64_t V, const uint1
  * D = 128, H / Hkv <= 4.  The workspace holds one int32 at
  * btl_decode_attention_error_offset (zero-filled before the first call): it
  * becomes non-zero when a position is outside [0, S) (that user's output is
- * then zero and its caches are not written).  Where B * Hkv pairs leave CUs
- * idle and S > 512, contexts are split over several workgroups, whose arrival
- * counters (zero between calls) and partials lie behind it: zero-fill the
- * whole workspace, and order the calls that share one. */
+ * then zero and its caches are not written).
+ *
+ * btl_decode_attention_split: the same with contexts split over several
+ * workgroups where B * Hkv pairs leave CUs idle and S > 512 (partials merged in
+ * a fixed order in fp32; a context that is not split gives the same bits).  split is a
+ * scratch of btl_decode_attention_split_bytes (0: no call of this shape splits),
+ * 16-byte aligned, zero-filled before its first call and not written
+ * by the caller between calls; calls that share one must not run at once (use one
+ * per cache: calls on one cache are ordered in any case).  A NULL split never splits. */
 int64_t btl_decode_attention_workspace_bytes(int64_t B, int64_t H, int64_t Hkv, int64_t S);
 int64_t btl_decode_attention_error_offset(int64_t B, int64_t Hkv);
 int btl_decode_attention(const uint16_t* qkv, int64_t B, int64_t H, int64_t Hkv, int64_t D, int64_t S,
                          const int32_t* pos, const float* rope_cos, const float* rope_sin, int rope_adjacent,
                          float scale, uint16_t* k_cache, uint16_t* v_cache, uint16_t* out, void* workspace,
                          size_t workspace_bytes, btl_stream_t stream);
+int64_t btl_decode_attention_split_bytes(int64_t B, int64_t Hkv, int64_t S);
+int btl_decode_attention_split(const uint16_t* qkv, int64_t B, int64_t H, int64_t Hkv, int64_t D, int64_t S,
+                               const int32_t* pos, const float* rope_cos, const float* rope_sin, int rope_adjacent,
+                               float scale, uint16_t* k_cache, uint16_t* v_cache, uint16_t* out, void* workspace,
+                               size_t workspace_bytes, void* split, size_t split_bytes, btl_stream_t stream);
 
 #ifdef __cplusplus
 }

@@ -374,6 +374,28 @@ def test_lm_head_sizes_and_argument_checks(L):
     assert L.btl_lm_head_repack(FAKE, 100, 250, FAKE, None) == SHAPE
 
 
+def test_decode_attention_keeps_its_one_word_workspace(L):
+    """btl_decode_attention's workspace is the error word (256 bytes) at every
+    shape, zeroed by its 4 bytes alone: what contexts split over workgroups
+    need is a scratch of the split entry's own query and arguments."""
+    shapes = [(1, 20, 5, 4096), (2, 20, 5, 4096), (22, 20, 5, 640), (32, 20, 5, 4096), (1, 4, 1, 512), (3, 8, 8, 1 << 20)]
+    for b, h, hkv, s in shapes:
+        assert L.btl_decode_attention_workspace_bytes(b, h, hkv, s) == 256, (b, h, hkv, s)
+    assert L.btl_decode_attention_split_bytes(2, 5, 4096) > 2 * 5 * 8 * 4 * 128 * 4
+    assert L.btl_decode_attention_split_bytes(32, 5, 4096) == 0  # 160 pairs: one workgroup each
+    assert L.btl_decode_attention_split_bytes(1, 5, 512) == 0  # one round of positions
+    assert L.btl_decode_attention_split_bytes(0, 5, 4096) == 0
+
+    def call(split=None, nbytes=0, ws_bytes=256, b=2, out=FAKE):
+        return L.btl_decode_attention_split(FAKE, b, 20, 5, 128, 4096, FAKE, FAKE, FAKE, 0, 0.1, FAKE, FAKE, out, FAKE,
+                                            ws_bytes, split, nbytes, None)
+
+    assert call(b=0) == 2 and call(out=None) == 1
+    assert call(ws_bytes=255) == 4
+    assert call(split=FAKE, nbytes=L.btl_decode_attention_split_bytes(2, 5, 4096) - 1) == 4
+    assert call(split=FAKE + 8, nbytes=1 << 20) == 3
+
+
 def test_weight_quant_pack_argument_checks(L):
     """The one-pass load refuses what the three passes refuse: NULL (1), shapes
     that are no multiples of 32 or too large (2), misalignment (3), a short

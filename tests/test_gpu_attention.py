@@ -372,6 +372,88 @@ def test_split_contexts(orc, B, Hq, Hkv, S, pos):
         check(orc, got, ref, cache, kc2, vc2)
 
 
+def test_whole_context_entry_needs_one_zero_word(orc):
+    """btl_decode_attention at a shape whose contexts the split entry would
+    split: a 256-byte workspace of which only the error word is zero."""
+    B, Hq, Hkv, S, D = 2, 20, 5, 2048, 128
+    pos = [2047, 1300]
+    att, cache, _, ref, kc, vc, kc2, vc2 = run(orc, B, Hq, Hkv, S, pos, False, 53)
+    rng = np.random.default_rng(53)
+    qkv = H.to_dev_bf16(orc.f32_to_bf16(rng.standard_normal((B, (Hq + 2 * Hkv) * D)).astype(np.float32)))
+    ws = torch.full((256,), 0xA5, dtype=torch.uint8, device=H.dev())
+    ws[:4] = 0
+    p = torch.tensor(pos, dtype=torch.int32, device=H.dev())
+    out = torch.full((B, Hq * D), 7.0, dtype=torch.bfloat16, device=H.dev())
+    N.check(N.lib().btl_decode_attention(
+        N.ptr(qkv), B, Hq, Hkv, D, S, N.ptr(p), N.ptr(att.rope_cos), N.ptr(att.rope_sin), 0, att.scale,
+        N.ptr(cache.key_cache), N.ptr(cache.value_cache), N.ptr(out), N.ptr(ws), 256, N.stream_of(H.dev())), "attention")
+    torch.cuda.synchronize()
+    assert int(ws[:4].view(torch.int32).item()) == 0 and bool((ws[4:] == 0xA5).all())
+    check(orc, H.bits_of(out), ref, cache, kc2, vc2)
+    # a cache object without a split scratch: the same whole contexts
+    cache.split = None
+    assert np.array_equal(H.bits_of(att(qkv, cache, p)), H.bits_of(out))
+
+
+def test_split_call_recovers_from_left_over_arrivals(orc):
+    """Arrivals that an earlier call left in the scratch do not keep a later
+    call from merging: the same bits as on a clean scratch, and the counts are
+    zero again."""
+    B, Hq, Hkv, S = 3, 20, 5, 4096
+    rng = np.random.default_rng(54)
+    att = DecodeAttention(Hq, Hkv, 128, S, H.dev())
+    cache = att.new_cache(B)
+    cache.key_cache.normal_()
+    cache.value_cache.normal_()
+    qkv = H.to_dev_bf16(orc.f32_to_bf16(rng.standard_normal((B, (Hq + 2 * Hkv) * 128)).astype(np.float32)))
+    pos = torch.tensor([4095, 700, 2000], dtype=torch.int32, device=H.dev())
+    ref = att(qkv, cache, pos)
+    words = cache.split[: 8 * B * Hkv].view(torch.int64)
+    words += torch.arange(B * Hkv, device=H.dev()) % 9
+    for rep in range(3):
+        out = torch.full_like(ref, 7.0)
+        att(qkv, cache, pos, out=out)
+        assert torch.equal(out, ref), rep
+        assert int((words % 16).abs().max().item()) == 0, rep
+
+
+def test_graphs_of_one_stream_replayed_at_once(orc):
+    """Two graphs captured on one stream, each with its own cache, replayed on
+    two streams at once give what each gives alone."""
+    B, Hq, Hkv, S = 2, 20, 5, 4096
+    att = DecodeAttention(Hq, Hkv, 128, S, H.dev())
+    s = torch.cuda.Stream()
+    calls = []
+    for i in range(2):
+        cache = att.new_cache(B)
+        cache.key_cache.normal_()
+        cache.value_cache.normal_()
+        qkv = torch.randn((B, (Hq + 2 * Hkv) * 128), device=H.dev()).bfloat16()
+        pos = torch.tensor([4000 - 900 * i, 3000], dtype=torch.int32, device=H.dev())
+        out = torch.empty((B, Hq * 128), dtype=torch.bfloat16, device=H.dev())
+        torch.cuda.synchronize()
+        with torch.cuda.stream(s):
+            att(qkv, cache, pos, out=out)
+        s.synchronize()
+        ref = out.clone()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s):
+            for _ in range(8):
+                att(qkv, cache, pos, out=out)
+        calls.append((g, out, ref, cache, qkv, pos, torch.cuda.Stream()))
+    for rep in range(20):
+        for g, out, *_ in calls:
+            out.zero_()
+        torch.cuda.synchronize()
+        for g, *_, st in calls:
+            with torch.cuda.stream(st):
+                g.replay()
+        torch.cuda.synchronize()
+        for i, (g, out, ref, *_) in enumerate(calls):
+            assert torch.equal(out, ref), (rep, i)
+    att.check()
+
+
 @pytest.mark.parametrize("batch,kv,S", [(1, 1, 4096), (5, 2, 1024), (26, 1, 640)])
 def test_persistent_full_step_split_contexts(orc, batch, kv, S):
     """The one-launch step with split contexts against step_full, bit for bit,
