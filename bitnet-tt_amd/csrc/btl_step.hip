@@ -1004,9 +1004,9 @@ __device__ void step_gemm_op(const StepArgs& p, const StepOp* sops, int l, int g
 // LDS: the unit index (read back each layer) and a zero (read by the attention).
 constexpr int kStepIdxInt = 20400;
 // Decode attention item ai of the layer (ATT instances; src/bitnet_tt/
-// inference/generator_batch32.py:728-746): split ai / (M Hkv) of pair
-// ai % (M Hkv), user b and key-value head hk, run by a GEMM workgroup between its QKV
-// and o_proj units.  The first round of the pair's cached keys and values does
+// inference/generator_batch32.py:728-746): split smax - 1 - ai / (M Hkv) of
+// pair ai % (M Hkv), user b and key-value head hk, run by a GEMM workgroup
+// between its QKV and o_proj units.  The first round of the pair's cached keys and values does
 // not depend on this step, so its loads are issued first; then the new token's
 // rows (the group's G query heads, and for split 0 its key and value head)
 // come in as row b's tagged QKV output words, and the body shared with
@@ -1018,7 +1018,7 @@ constexpr int kStepIdxInt = 20400;
 // reused a layer later: its writer has then seen QKV words that depend on this
 // layer's attention output, so split 0 has read it.
 // Split 0's thread (g, d): its output from its own partial and the tagged
-// words of the other splits (items ai + i M Hkv).  Every load of a
+// words of the other splits (items ai - i M Hkv).  Every load of a
 // round is issued before a tag is checked.
 __device__ __forceinline__ uint32_t gather_partials(const StepArgs& p, const AttnSmem& s, int ai, int n,
                                                     const AttnPartial& mine, uint32_t want, WaitState& ws) {
@@ -1033,7 +1033,7 @@ __device__ __forceinline__ uint32_t gather_partials(const StepArgs& p, const Att
 #pragma unroll
     for (int i = 1; i < kAtMaxSplits; ++i)
       if (i < n) {
-        const uint64_t* const w = w0 + (int64_t)i * p.M * p.Hkv * kAtPartFloats;
+        const uint64_t* const w = w0 - (int64_t)i * p.M * p.Hkv * kAtPartFloats;
         o[i] = ld_coherent(w + tid);
         m[i] = ld_coherent(w + ml);
         l[i] = ld_coherent(w + ml + 1);
@@ -1069,7 +1069,7 @@ __device__ void step_attention(const StepArgs& p, int l, int ai, uint32_t E, int
   a.S = p.S;
   const int pairs = p.M * p.Hkv, pr = SPLIT ? ai % pairs : ai;
   a.smax = smax;
-  a.split = SPLIT ? ai / pairs : 0;
+  a.split = SPLIT ? smax - 1 - ai / pairs : 0;
   a.b = pr / p.Hkv;
   a.hk = pr % p.Hkv;
   a.pos = __builtin_amdgcn_readfirstlane(p.pos[a.b]);
@@ -1141,8 +1141,13 @@ __device__ void step_attention(const StepArgs& p, int l, int ai, uint32_t E, int
 
 
 // The first GEMM unit with an attention item: the items (smax per user and
-// key-value head) take the last units, which at the 2B shape (160 items, 60 QKV units of 224) have no QKV
-// work, so each issues its cached keys and values at the start of the layer.
+// key-value head) take the last units, the splits 0 the last of all.  Split 0
+// always has work and merges its pair; at the 2B shape (224 units, QKV on the
+// first 60, at most 160 pairs) its units have no QKV work, so each issues its
+// cached keys and values at the start of the layer.  With the splits 0 first
+// they fell on QKV units at 5 to 22 users and held a layer up by up to 5 us (5
+// users, cache of 4096, us a layer at position 300 / 2000 / 4000: 31.8 / 34.8 /
+// 36.6, now 26.7 / 32.6 / 36.4; 26.5 / 46.7 / 72.2 without the split).
 __device__ __forceinline__ int step_first_att(const StepArgs& p) {
   return (int)gridDim.x - kStepRows - p.M * p.Hkv * p.smax;
 }

@@ -479,6 +479,30 @@ def test_persistent_full_step_split_contexts(orc, batch, kv, S):
         _compare(_outputs(step), ref, f"split contexts, back {back}")
 
 
+@pytest.mark.parametrize("batch", [5, 11, 22])
+def test_persistent_full_step_split_contexts_on_qkv_units(orc, batch):
+    """Batches at the 2B shape whose attention items reach units that also run
+    QKV (200, 220 and 220 items of 224 units, 60 of them QKV's), users at short,
+    middle and long contexts: the one-launch step against step_full."""
+    from bitnet_tt.config import BitNet2B4TConfig
+    from bitnet_tt.decode import BitLinearDecodeStep
+
+    print(f"persistent full step, split contexts at the 2B shape: batch {batch}", flush=True)
+    step = BitLinearDecodeStep.random_init(BitNet2B4TConfig(), H.dev(), seed=87, batch=batch, num_layers=2)
+    step.alloc_buffers(seed=88).alloc_attention(max_seq_len=4096)
+    for first in (4095, 700):
+        step.pos.copy_(torch.tensor([max(0, first - 190 * i) for i in range(batch)], dtype=torch.int32))
+        state = _full_state(step)
+        step.step_full()
+        step.check()
+        ref = _outputs(step)
+        for rep in range(2):
+            _restore(step, state)
+            step.step_persistent_full()
+            step.check()
+            _compare(_outputs(step), ref, f"batch {batch}, first position {first}, rep {rep}")
+
+
 # Batch 1, whose step has a kernel of its own: whole and split contexts, two
 # chunks of F per thread, and a shape whose 216 units and 64 attention items do
 # not fit 256 workgroups (the two-hop kernel).
