@@ -184,7 +184,13 @@ __device__ __forceinline__ uint4 att_ld(__amdgpu_buffer_rsrc_t r, int voff, int 
   return make_uint4(v[0], v[1], v[2], v[3]);
 }
 
-// Keys and values of this wave's block `blk` of 64 positions.
+// Keys and values of this wave's block `blk` of 64 positions.  AHEAD: 28 of the
+// 32 loads are issued before anything that follows.  Left to itself the
+// compiler put half of a later round's loads in the one-launch step behind
+// waits for its first keys (32 users, cache of 4096, us a layer at position
+// 2000 / 4000: 55.5 / 85.5 against 52.7 / 80.8; 24 users' standalone call at 4000
+// 60.2 against 58.1); with all 32 ahead its instances spill 3 to 9 registers.
+template <bool AHEAD = false>
 __device__ __forceinline__ void att_load_block(const AttnPair& a, int blk, AttnRound& r) {
   const int lane = a.tid & 63, r16 = lane & 15, grp = lane >> 4, base = blk * kAtPosWave;
   const __amdgpu_buffer_rsrc_t kc = att_rows(a.kc, a), vc = att_rows(a.vc, a);
@@ -199,6 +205,7 @@ __device__ __forceinline__ void att_load_block(const AttnPair& a, int blk, AttnR
   for (int t = 0; t < 16; ++t) {
     const int row = min(base + 4 * t + grp, a.S - 1);
     r.vr[t] = att_ld(vc, (row * kAtD + 8 * r16) * 2, 0);
+    if (AHEAD && t == 11) __builtin_amdgcn_sched_barrier(0);
   }
 }
 
@@ -308,7 +315,7 @@ __device__ __forceinline__ uint16_t att_body(const AttnPair& a, AttnSmem& s, Att
   for (int rd = 0; rd < nrounds; ++rd) {
     const int blk = a.block0() + rd * kAtWaves + wv, base = kAtPosWave * blk;
     if (blk >= blk1) break;  // wave-uniform: nothing cached from here on
-    if (rd > 0) att_load_block(a, blk, r);
+    if (rd > 0) att_load_block<true>(a, blk, r);
     // scores: 4 blocks of 16 positions
     v4f sc[4];
 #pragma unroll
