@@ -40,14 +40,14 @@ struct AttnArgs {
   int B, H, Hkv, G, S;
   float scale;
   int adjacent;            // 1: RoPE pairs (2i, 2i+1); 0: (i, i + D/2)
-  int smax;                // workgroups per (user, key-value head)
-  // smax > 1.  A pair's arrival word is a call's number plus the splits that
+  AttnSplits sp;           // sp.smax workgroups per (user, key-value head)
+  // sp.smax > 1.  A pair's arrival word is a call's number plus the splits that
   // have arrived, which is zero between calls.  Every split raises the word to
   // its own call's number before it arrives, so that a count left over from two
   // calls that ran at once on one scratch does not outlive them.
   uint64_t* arrive;        // [pairs]
   uint64_t call;           // a multiple of kAttnCallStep, larger in each later call
-  float* part;             // [pairs][smax][kAtPartFloats]
+  float* part;             // [pairs][sp.smax][kAtPartFloats]
 };
 constexpr uint64_t kAttnCallStep = 16;  // > kAtMaxSplits
 static_assert(kAtMaxSplits < (int)kAttnCallStep, "arrivals fit below the call's number");
@@ -62,7 +62,7 @@ __device__ bool attn_gather(const AttnArgs& p, const AttnPair& a, int pair, int 
                             int* s_last, float (&Ms)[kAtMaxSplits], float (&Ls)[kAtMaxSplits],
                             float (&Os)[kAtMaxSplits]) {
   const int tid = threadIdx.x, g = tid / kAtD;
-  float* const base = p.part + (int64_t)pair * p.smax * kAtPartFloats;
+  float* const base = p.part + (int64_t)pair * p.sp.smax * kAtPartFloats;
   if (g < a.G) {
     float* const o = base + a.split * kAtPartFloats;
     st_coherent(o + tid, mine.O);
@@ -93,7 +93,7 @@ __device__ bool attn_gather(const AttnArgs& p, const AttnPair& a, int pair, int 
   return true;
 }
 
-// SPLIT: smax > 1 workgroups per pair.
+// SPLIT: sp.smax > 1 workgroups per pair.
 template <bool SPLIT>
 __global__ __launch_bounds__(64 * kAtWaves, 1) void k_decode_attention(AttnArgs p) {
   __shared__ __attribute__((aligned(16))) AttnSmem s;
@@ -108,21 +108,19 @@ __global__ __launch_bounds__(64 * kAtWaves, 1) void k_decode_attention(AttnArgs 
   a.Hkv = p.Hkv;
   a.G = p.G;
   a.S = p.S;
-  // every pair's split 0 first: they are spread over the XCDs, and where a
-  // context is one round they do not queue behind workgroups that only leave
-  const int pairs = p.B * p.Hkv;
-  const int pair = SPLIT ? blockIdx.x % pairs : blockIdx.x;
-  a.smax = SPLIT ? p.smax : 1;
-  a.split = SPLIT ? blockIdx.x / pairs : 0;
-  a.hk = pair % p.Hkv;
-  a.b = pair / p.Hkv;
-  a.pos = __builtin_amdgcn_readfirstlane(p.pos[a.b]);
+  // grid (Hkv, B, splits), so no index needs a division; every pair's split 0
+  // first: they are spread over the XCDs, and where a context is one round they
+  // do not queue behind workgroups that only leave
+  a.hk = blockIdx.x;
+  a.b = blockIdx.y;
+  a.split = SPLIT ? blockIdx.z : 0;
+  a.sp = SPLIT ? p.sp : AttnSplits{1, 0};
+  const int pair = a.b * p.Hkv + a.hk;
   a.scale = p.scale;
   a.adjacent = p.adjacent;
   a.tid = tid;
-  if (a.split != 0 && a.split >= a.splits()) return;
   AttnRound r;
-  att_load_first(a, r);
+  if (!att_load_first<true>(a, p.pos + a.b, r)) return;
   BTL_TRACE_AT(1);
   if (!a.pos_ok() && tid == 0 && a.hk == 0 && a.split == 0) st_coherent(p.error, 1);
   // the new token's rows of the group: q rows hk G .. hk G + G - 1, k row hk, v row hk
@@ -136,7 +134,7 @@ __global__ __launch_bounds__(64 * kAtWaves, 1) void k_decode_attention(AttnArgs 
   __syncthreads();
   BTL_TRACE_AT(2);
   AttnPartial part;
-  const int n = SPLIT ? a.splits() : 1;
+  const int n = SPLIT ? a.n : 1;
   // long before this split's own arrival, which waits for it
   if (SPLIT && n > 1 && tid == 0) atomicMax(reinterpret_cast<unsigned long long*>(p.arrive + pair), p.call);
   uint16_t o = att_body(a, s, r, part, true);
@@ -215,17 +213,17 @@ static int decode_attention(const char* who, const uint16_t* qkv, int64_t B, int
   a.scale = scale;
   a.adjacent = rope_adjacent ? 1 : 0;
   a.error = reinterpret_cast<int32_t*>(workspace);
-  a.smax = split ? att_max_splits(B * Hkv, S, device_cus()) : 1;
+  a.sp = split ? att_splits(B, H, Hkv, S, device_cus()) : AttnSplits{1, 0};
   a.arrive = nullptr;
   a.call = 0;
   a.part = nullptr;
-  if (a.smax > 1) {
+  if (a.sp.smax > 1) {
     a.arrive = reinterpret_cast<uint64_t*>(split);
     a.call = kAttnCallStep * (calls.fetch_add(1, std::memory_order_relaxed) + 1);
     a.part = reinterpret_cast<float*>(static_cast<char*>(split) + kAttnPart);
   }
-  const dim3 grid((unsigned)(B * Hkv * a.smax));
-  if (a.smax > 1)
+  const dim3 grid((unsigned)Hkv, (unsigned)B, (unsigned)a.sp.smax);
+  if (a.sp.smax > 1)
     hipLaunchKernelGGL(k_decode_attention<true>, grid, dim3(64 * kAtWaves), 0, (hipStream_t)stream, a);
   else
     hipLaunchKernelGGL(k_decode_attention<false>, grid, dim3(64 * kAtWaves), 0, (hipStream_t)stream, a);

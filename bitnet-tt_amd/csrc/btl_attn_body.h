@@ -60,14 +60,25 @@ constexpr int kAtMinBlocks = 4;                  // blocks of 64 positions a spl
 constexpr int kAtSplitItems = 224;
 constexpr int kAtPartFloats = kAtMaxG * kAtD + 2 * kAtMaxG;  // one split's partial: outputs, maxima, sums
 
-// Most splits per pair: one where the pairs alone fill the chip or the cache
-// is a single round.  Measured on MI355X (20 / 5 heads, cache of 4096, one
-// workgroup a pair -> split, us a launch): 1 user at 640 / 2048 / 4096
-// positions 11.6 -> 11.0, 26.5 -> 11.4, 50.4 -> 13.6; 8 users 12.5 -> 12.0,
-// 27.8 -> 14.8, 56.4 -> 23.3; 22 users 13.1 -> 14.4, 36.2 -> 27.6, 66.3 ->
-// 47.3.  Up to 512 positions a context stays whole (10.2 us; the workgroups
-// that find nothing to do cost 0.5 us).  Eight splits and not sixteen: with
-// the words of sixteen the one-launch step's instance spills.
+// How the contexts of a call are split.  smax, the most splits per pair: one
+// where the pairs alone fill the chip or the cache is a single round.  Eight
+// splits and not sixteen: with the words of sixteen the one-launch step's
+// instance spills.  first: a context of up to this many blocks of 64 positions
+// stays whole.  One round always does; where at most three splits share a
+// context and the step has to put some of them on units that run QKV as well
+// (2 per head of the 2B shape's NQKV / 64), which get to them 3 us late, up to
+// 14 (three splits) or 20 blocks.
+// Measured on MI355X (20 / 5 heads, cache of 4096; whole -> split).  The
+// standalone launch, us: 1 user at 640 / 2000 / 4000 positions 11.6 -> 10.7,
+// 26.6 -> 11.1, 50.0 -> 12.7; 8 users 12.4 -> 11.3, 27.5 -> 13.5, 55.4 -> 21.1; 22 users
+// 13.0 -> 13.8, 31.9 -> 25.7, 59.6 -> 44.2.  The step, us a layer: 8 users 29.8 -> 28.0,
+// 47.4 -> 32.8, 73.2 -> 41.4; 14 users at 640 / 768 / 1000 30.8 -> 31.6, 31.8 -> 32.7, 34.7
+// -> 33.0; 16 users (no split on a QKV unit) at 640 31.0 -> 29.1; 17 users at 640 / 1152 /
+// 1500 31.2 -> 33.1, 37.6 -> 38.4, 42.7 -> 39.7; 22 users 31.7 -> 33.9, 38.7 -> 40.1, 44.0
+// -> 41.7.  A context that stays whole costs 0.2 to 0.4 us more in the split launch.
+struct AttnSplits {
+  int smax, first;
+};
 inline int att_max_splits(int64_t pairs, int64_t S, int64_t cus) {
   int64_t n = (cus - 32 < kAtSplitItems ? cus - 32 : kAtSplitItems) / pairs;
   const int64_t blocks = (S + kAtPosWave - 1) / kAtPosWave;
@@ -75,6 +86,11 @@ inline int att_max_splits(int64_t pairs, int64_t S, int64_t cus) {
   if (n > blocks / kAtMinBlocks) n = blocks / kAtMinBlocks;
   if (n > kAtMaxSplits) n = kAtMaxSplits;
   return n > 1 ? (int)n : 1;
+}
+inline AttnSplits att_splits(int64_t B, int64_t H, int64_t Hkv, int64_t S, int64_t cus) {
+  const int n = att_max_splits(B * Hkv, S, cus);
+  const bool on_qkv = B * Hkv * n > kAtSplitItems - 2 * (H + 2 * Hkv);
+  return {n, !on_qkv || n > 3 ? kAtWaves : n == 3 ? 14 : 20};
 }
 
 struct AttnSmem {
@@ -97,7 +113,8 @@ struct AttnPair {
   uint16_t* kc;       // [B, Hkv, S, D]
   uint16_t* vc;
   int Hkv, G, S, b, hk, pos;
-  int smax, split;    // most splits of the pair (att_max_splits), this workgroup's
+  AttnSplits sp;      // smax 1: whole contexts
+  int split;          // this workgroup's
   float scale;
   int adjacent;  // 1: RoPE pairs (2i, 2i+1); 0: (i, i + D/2)
   // This thread's index in the workgroup.  A caller that runs the body inside
@@ -107,19 +124,25 @@ struct AttnPair {
   int tid;
   __device__ __forceinline__ bool pos_ok() const { return pos >= 0 && pos < S; }
   __device__ __forceinline__ int nold() const { return pos_ok() ? pos : 0; }  // cached positions [0, nold)
-  // The pair's blocks of 64 cached positions, how many a split takes, the
-  // splits that have any, and this split's range of blocks.
-  __device__ __forceinline__ int blocks() const { return (nold() + kAtPosWave - 1) / kAtPosWave; }
-  __device__ __forceinline__ int per_split() const {
-    const int nb = blocks();
-    return smax == 1 || nb <= kAtWaves ? nb : max(kAtMinBlocks, (nb + smax - 1) / smax);
+  // The splits of the pair's context that have any of its blocks of 64 cached
+  // positions, and this split's range of blocks [blk0, blk1) (empty where it
+  // has none): from the position, by plan().
+  int n, blk0, blk1;
+  __device__ __forceinline__ void plan() {
+    const int nb = (nold() + kAtPosWave - 1) / kAtPosWave;
+    n = 1;
+    blk0 = 0;
+    blk1 = nb;
+    if (sp.smax == 1) return;
+    if (nb > sp.first) {
+      const int per = max(kAtMinBlocks, (nb + sp.smax - 1) / sp.smax);
+      n = (nb + per - 1) / per;
+      blk0 = split * per;
+      blk1 = min(nb, blk0 + per);
+    } else if (split != 0) {
+      blk0 = nb;
+    }
   }
-  __device__ __forceinline__ int splits() const {
-    const int nb = blocks(), per = per_split();
-    return nb == per ? 1 : (nb + per - 1) / per;
-  }
-  __device__ __forceinline__ int block0() const { return split == 0 ? 0 : split * per_split(); }
-  __device__ __forceinline__ int block1() const { return min(blocks(), block0() + per_split()); }
   __device__ __forceinline__ int64_t kv_base() const { return ((int64_t)b * Hkv + hk) * S; }
 };
 
@@ -209,22 +232,42 @@ __device__ __forceinline__ void att_load_block(const AttnPair& a, int blk, AttnR
   }
 }
 
-// The first round, then the RoPE factors of frequency tid & 63 at the
-// position.  Split 0's first blocks do not depend on the position, which may
-// itself still be on its way (waiting for it first costs 1 us a launch); in
-// the other splits a wave with no block loads none.
-__device__ __forceinline__ void att_load_first(const AttnPair& a, AttnRound& r) {
+// The first round, the position (a.pos, a.plan) and the RoPE factors of
+// frequency tid & 63 at it; false for a split with nothing to do.  In the
+// splits but the first a wave with no block loads none.  EARLY (the standalone
+// launch): the first blocks of a whole context or of split 0, which do not
+// depend on the position, do not wait for it either (0.5 us a launch).  In the
+// one-launch step they are not what the layer waits for, and the plain order
+// is up to 1 us a layer faster there (batch 1).
+template <bool EARLY>
+__device__ __forceinline__ bool att_load_first(AttnPair& a, const int32_t* pos, AttnRound& r) {
   const int wv = __builtin_amdgcn_readfirstlane(a.tid >> 6);
+  // EARLY: the position is asked for ahead of the first blocks, and after
+  // everything that their loads need (the zero index depends on it): a wait
+  // for one scalar load is a wait for all.
+  int zero = 0;
+  if (EARLY) asm("s_mov_b32 %0, 0" : "=s"(zero) : "s"(a.kc), "s"(a.vc), "s"(a.S), "s"(a.Hkv));
+  const int apos = pos[zero];
   int blk = wv;
   bool any = true;
-  if (a.split != 0) {
-    blk += a.split * a.per_split();
-    any = blk < a.block1();
+  if (!EARLY || a.split != 0) {
+    a.pos = __builtin_amdgcn_readfirstlane(apos);
+    a.plan();
+    if (a.split != 0) {
+      if (a.blk0 >= a.blk1) return false;
+      blk += a.blk0;
+      any = blk < a.blk1;
+    }
   }
   if (any) att_load_block(a, blk, r);
+  if (EARLY) {
+    a.pos = __builtin_amdgcn_readfirstlane(apos);
+    a.plan();
+  }
   const int i = a.tid & (kAtD / 2 - 1), pc = a.pos_ok() ? a.pos : 0;
   r.rc = a.rcos[pc * (kAtD / 2) + i];
   r.rs = a.rsin[pc * (kAtD / 2) + i];
+  return true;
 }
 
 // A thread's share of a split's partial: head tid / D, dimension tid % D.
@@ -252,7 +295,6 @@ __device__ __forceinline__ uint16_t att_body(const AttnPair& a, AttnSmem& s, Att
   const int G = a.G;
   const bool pos_ok = a.pos_ok();
   const int nold = a.nold();
-  const int blk1 = a.block1();
   const int64_t kvb = a.kv_base();
   const int half = kAtD / 2;
   const int r16 = lane & 15, grp = lane >> 4;
@@ -311,10 +353,10 @@ __device__ __forceinline__ uint16_t att_body(const AttnPair& a, AttnSmem& s, Att
 #pragma unroll
   for (int m = 0; m < kAtD / 16; ++m) o[m] = (v4f){0.f, 0.f, 0.f, 0.f};
 
-  const int nrounds = (blk1 - a.block0() + kAtWaves - 1) / kAtWaves;
+  const int nrounds = (a.blk1 - a.blk0 + kAtWaves - 1) / kAtWaves;
   for (int rd = 0; rd < nrounds; ++rd) {
-    const int blk = a.block0() + rd * kAtWaves + wv, base = kAtPosWave * blk;
-    if (blk >= blk1) break;  // wave-uniform: nothing cached from here on
+    const int blk = a.blk0 + rd * kAtWaves + wv, base = kAtPosWave * blk;
+    if (blk >= a.blk1) break;  // wave-uniform: nothing cached from here on
     if (rd > 0) att_load_block<true>(a, blk, r);
     // scores: 4 blocks of 16 positions
     v4f sc[4];
@@ -416,7 +458,7 @@ __device__ __forceinline__ uint16_t att_body(const AttnPair& a, AttnSmem& s, Att
   uint16_t res = 0;
   {
     const int g = tid / kAtD, d = tid % kAtD;  // 512 threads: 4 heads x 128 dims
-    if (g < G && a.splits() > 1) {
+    if (g < G && a.n > 1) {
       float M = -__builtin_inff();
 #pragma unroll
       for (int w = 0; w < kAtWaves; ++w) M = fmaxf(M, s.ml[w][g][0]);

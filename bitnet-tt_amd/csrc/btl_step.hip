@@ -189,7 +189,11 @@ struct StepArgs {
   uint16_t* attn_out;
   int64_t off_att;
   int64_t off_part;  // the attention splits' partials as tagged words, one slot per item
-  int Hkv, G, S, adjacent, smax;
+  int Hkv, G, S, adjacent;
+  // AttnSplits as smax + 16 first: one word, since with two more the one-user
+  // kernel spills scalar registers and takes 0.7 us more a layer.
+  int splits;
+  __device__ __forceinline__ AttnSplits sp() const { return {splits & 15, splits >> 4}; }
   float scale;
 };
 
@@ -1055,7 +1059,7 @@ __device__ __forceinline__ uint32_t gather_partials(const StepArgs& p, const Att
 
 template <bool SPLIT>
 __device__ void step_attention(const StepArgs& p, int l, int ai, uint32_t E, int32_t* lds, WaitState& ws) {
-  const int smax = SPLIT ? p.smax : 1;
+  const int smax = SPLIT ? p.sp().smax : 1;
   if (ai < 0 || ai >= p.M * p.Hkv * smax) return;
   const int tid = threadIdx.x;
   AttnSmem& s = *reinterpret_cast<AttnSmem*>(lds);
@@ -1068,22 +1072,20 @@ __device__ void step_attention(const StepArgs& p, int l, int ai, uint32_t E, int
   a.G = p.G;
   a.S = p.S;
   const int pairs = p.M * p.Hkv, pr = SPLIT ? ai % pairs : ai;
-  a.smax = smax;
+  a.sp = SPLIT ? p.sp() : AttnSplits{1, 0};
   a.split = SPLIT ? smax - 1 - ai / pairs : 0;
   a.b = pr / p.Hkv;
   a.hk = pr % p.Hkv;
-  a.pos = __builtin_amdgcn_readfirstlane(p.pos[a.b]);
   a.scale = p.scale;
   a.adjacent = p.adjacent;
   // the thread index plus a zero read back from LDS on every call: the body's
   // per-lane values are recomputed in each layer rather than kept (spilled)
   // across the layer loop
   a.tid = tid + *reinterpret_cast<volatile int32_t*>(lds + kStepIdxInt + 1);
-  const int nsplits = SPLIT ? a.splits() : 1;
-  if (a.split != 0 && a.split >= nsplits) return;  // uniform: every thread holds the same position
-  if (!a.pos_ok() && tid == 0) set_error_word(p, BAD_POSITION, (uint32_t)(l * 4 + S_O));
   AttnRound r;
-  att_load_first(a, r);
+  if (!att_load_first<false>(a, p.pos + a.b, r)) return;  // uniform: every thread holds the same position
+  const int nsplits = SPLIT ? a.n : 1;
+  if (!a.pos_ok() && tid == 0) set_error_word(p, BAD_POSITION, (uint32_t)(l * 4 + S_O));
   STEP_TRACE(l, 0);
   // the new rows: thread t < 6 x 64 takes word t % 64 (two values) of row
   // segment t / 64 (query rows 0..G-1, the key row at kAtMaxG, the value row
@@ -1149,7 +1151,7 @@ __device__ void step_attention(const StepArgs& p, int l, int ai, uint32_t E, int
 // users, cache of 4096, us a layer at position 300 / 2000 / 4000: 31.8 / 34.8 /
 // 36.6, now 26.7 / 32.6 / 36.4; 26.5 / 46.7 / 72.2 without the split).
 __device__ __forceinline__ int step_first_att(const StepArgs& p) {
-  return (int)gridDim.x - kStepRows - p.M * p.Hkv * p.smax;
+  return (int)gridDim.x - kStepRows - p.M * p.Hkv * p.sp().smax;
 }
 
 // NQ: superblocks per wave of a unit of QKV, O and GU (K = H); NDN: of DN
@@ -1431,7 +1433,7 @@ __global__ __launch_bounds__(512) void k_decode_step_one(StepArgs p) {
   const uint32_t E = p.epoch[u] + 1u;
   WaitState ws{false, false};
   if (ATT) {
-    const int ai = u - ((int)gridDim.x - p.Hkv * (ATT == 2 ? p.smax : 1));
+    const int ai = u - ((int)gridDim.x - p.Hkv * (ATT == 2 ? p.sp().smax : 1));
     if (ai >= 0) {  // an attention workgroup: no unit, so its caches travel from the layer's start
       for (int l = 0; l < p.L; ++l) step_attention<ATT == 2>(p, l, ai, E, lds, ws);
       if (tid == 0) p.epoch[u] = E;
@@ -1733,7 +1735,7 @@ static int launch_step(const StepArgs& a, int64_t F, int att, const char* who, h
   // One user: the kernel whose units do the row work themselves, where the
   // attention items leave every unit a workgroup of its own.
   const int64_t units = std::max({a.NQKV / 32, a.H / 32, a.F / 32});
-  const int64_t items = att ? (int64_t)a.Hkv * a.smax : 0;
+  const int64_t items = att ? (int64_t)a.Hkv * (a.splits & 15) : 0;
   const bool one = a.M == 1 && units + items <= step_grid();
   void (*k)(StepArgs) = one ? step_one_fn(F, att) : step_kernel_fn(F, att);
   if (!k) return set_error(BTL_ERR_SHAPE, "%s: no kernel instance for F=%lld", who, (long long)F);
@@ -1916,13 +1918,14 @@ int btl_decode_step_full(int64_t M, int64_t H, int64_t F, int64_t NQKV, int64_t 
   a.attn_out = attn_out;
   a.off_att = z.off_att;
   a.off_part = z.off_part;
-  a.smax = att_max_splits(M * Hkv, S, step_grid());
+  const AttnSplits sp = att_splits(M, Hq, Hkv, S, step_grid());
+  a.splits = sp.smax + 16 * sp.first;
   a.Hkv = (int)Hkv;
   a.G = (int)(Hq / Hkv);
   a.S = (int)S;
   a.adjacent = rope_adjacent ? 1 : 0;
   a.scale = scale;
-  return launch_step(a, F, a.smax > 1 ? 2 : 1, "btl_decode_step_full", (hipStream_t)stream);
+  return launch_step(a, F, sp.smax > 1 ? 2 : 1, "btl_decode_step_full", (hipStream_t)stream);
 }
 
 int btl_decode_step_floor(int64_t M, int64_t H, int64_t F, int64_t NQKV, int64_t L, void* workspace,

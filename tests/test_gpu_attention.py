@@ -348,8 +348,9 @@ def test_persistent_full_step_matches_step_full_2b(orc):
 
 
 # (users, query heads, kv heads, cache length, positions): the edges of one
-# round (511..513 cached positions), of the blocks of 64 and of the splits'
-# ranges; 8, 5, 2 and 1 splits per pair; an out-of-range user among split ones
+# round (511..513 cached positions), of the blocks of 64, of the splits'
+# ranges and of the contexts that stay whole (896 and 1280 positions at 13 and 20
+# users); 8, 5, 3, 2 and 1 splits per pair; an out-of-range user among split ones
 # is left to test_position_out_of_range_is_flagged's single-split shape.
 SPLIT_SHAPES = [
     (1, 4, 1, 4096, [4095]),
@@ -358,6 +359,8 @@ SPLIT_SHAPES = [
     (3, 8, 8, 1000, [999, 640, 513]),
     (16, 20, 5, 1024, [1023 - 37 * i for i in range(16)]),
     (23, 20, 5, 640, [639 - i for i in range(23)]),
+    (13, 20, 5, 1024, [895, 896, 897, 960, 961, 1023, 512, 513, 0, 1, 700, 64, 1000]),
+    (20, 20, 5, 1400, [1279, 1280, 1281, 1399, 1344, 1345, 640, 513, 512, 0] + [1390 - 70 * i for i in range(10)]),
 ]
 
 
@@ -479,10 +482,10 @@ def test_persistent_full_step_split_contexts(orc, batch, kv, S):
         _compare(_outputs(step), ref, f"split contexts, back {back}")
 
 
-@pytest.mark.parametrize("batch", [5, 11, 22])
+@pytest.mark.parametrize("batch", [5, 11, 13, 22])
 def test_persistent_full_step_split_contexts_on_qkv_units(orc, batch):
     """Batches at the 2B shape whose attention items reach units that also run
-    QKV (200, 220 and 220 items of 224 units, 60 of them QKV's), users at short,
+    QKV (200, 220, 195 and 220 items of 224 units, 60 of them QKV's), users at short,
     middle and long contexts: the one-launch step against step_full."""
     from bitnet_tt.config import BitNet2B4TConfig
     from bitnet_tt.decode import BitLinearDecodeStep
