@@ -189,16 +189,18 @@ __global__ __launch_bounds__(64 * kActRowWaves) void k_act_rows_wave(ActArgs p) 
 template <bool NORM, bool QUANT>
 static void launch_rows(unsigned rows, hipStream_t s, const ActArgs& p) {
   // rows is a multiple of 32 (whole row blocks) when quantising.  From 256 rows
-  // four waves a row; one wave from 1536 rows where it can skip blocks of the
-  // row past K (K <= 2560: five of eight in use); the 512-thread row below 256.
-  // Measured on MI355X, graph-timed, one / two / four waves a row (us):
-  // K = 2560, M = 256 / 511 / 1024 / 2048: - / 4.37 / 3.72, - / 4.52 / 4.14, 5.51 /
-  // 5.25 / 5.42, 7.97 / 8.79 / 8.55; K = 6912: - / 5.66 / 4.44, - / 6.33 / 5.75,
-  // 10.5 / 9.7 / 9.0, 15.2 / 14.2 / 13.5; K = 4096, M = 2048: 11.1 / 9.8 / 9.8; M = 100
-  // in 512-thread rows 3.65 (K = 2560), 4.4 (6912).
+  // four waves a row; one wave where it can skip blocks of the row past K (four
+  // or five of eight in use) and the rows alone fill the chip: from 896 rows up
+  // to K = 2048, from 1536 rows up to 2560; the 512-thread row below 256.
+  // Measured on MI355X, graph-timed, one / four waves a row (us): M = 768 / 896 /
+  // 1280 / 2048 at K = 256: 3.9 / 4.2, 4.0 / 4.7, 4.1 / 5.1, 4.2 / 6.5; K = 1024: 4.3 / 4.4, 4.3 / 5.0,
+  // 4.6 / 5.4, 4.7 / 7.0; K = 2048: 5.0 / 4.5, 5.0 / 5.2, 5.6 / 5.7, 6.7 / 7.9; M = 896 / 1280 / 1536 /
+  // 2048 at K = 2560: 5.4 / 5.3, 6.2 / 5.9, 6.9 / 7.0, 7.9 / 8.4; K = 3072: 5.7 / 5.3, 7.5 / 6.6, 8.2 /
+  // 7.6, 8.8 / 8.7; K = 6912: 9.8 / 8.7, 12.8 / 9.9, 13.2 / 10.9, 14.6 / 13.1.  M = 128 in 512-thread
+  // rows 3.6 (K = 2560), 4.4 (6912).
   if (QUANT && act_cpt(p.K) <= 2 && rows >= 256) {
     const dim3 block(64 * kActRowWaves);
-    if (p.K <= 2560 && rows >= 1536)
+    if (p.K <= 2560 && rows >= (p.K <= 2048 ? 896u : 1536u))
       hipLaunchKernelGGL((k_act_rows_wave<NORM, 1, 1>), dim3(rows / kActRowWaves), block, 0, s, p);
     else if (act_cpt(p.K) == 1)
       hipLaunchKernelGGL((k_act_rows_wave<NORM, 1, kActRowWaves>), dim3(rows), block, 0, s, p);

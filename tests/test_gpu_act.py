@@ -60,11 +60,12 @@ def test_quant_absmax_bit_exact(orc, m, k, norm):
 
 
 @pytest.mark.parametrize("m,k", [(225, 2560), (256, 64), (257, 8192), (400, 4128), (1504, 2560), (1505, 2560),
-                                 (1601, 2528), (1550, 32), (1540, 2592)])
+                                 (1601, 2528), (1550, 32), (1540, 2592), (300, 4096), (864, 2048), (865, 2048),
+                                 (900, 2080), (1000, 256)])
 def test_quant_absmax_wave_kernels(orc, m, k):
     """Edges of the wave-per-row kernels (M = 225 is the first row count in 256
-    padded rows, 1505 the first in 1536; K = 2560 the last one-wave width, 4096
-    and 8192 the last of one and two chunks a thread), norm on, against the
+    padded rows, 865 the first in 896 and 1505 in 1536, where one wave a row takes
+    over up to K = 2048 and 2560; 4096 and 8192 the last of one and two chunks a thread), norm on, against the
     oracle: codes, scales and row sums to the bit."""
     print(f"quant wave kernels m={m} k={k}", flush=True)
     xb = H.activations(orc, m, k, seed=m * 7 + k)
