@@ -85,6 +85,7 @@ EXPORTS = {
     "btl_gemm_tiling": ([_I64, _I64, _I64, _I, _I, _P], _I),
     "btl_gemm_workspace_bytes": ([_I64, _I64, _I64, _I, _I], _I64),
     "btl_fused_workspace_bytes": ([_I64, _I64, _I64, _I, _I], _I64),
+    "btl_fused_prefill_form": ([_I64, _I64, _I64, _I], _I),
     "btl_fused_error_offset": ([], _I64),
     "btl_weight_quant_scratch_bytes": ([_I64], _I64),
     "btl_weight_quant_ternary": ([_P, _I64, _F, _P, _P, _P, _SZ, _P], _I),

@@ -1744,16 +1744,26 @@ static void launch_prefill_epi(bool prs, int rb, bool sk, dim3 grid, hipStream_t
 // Which k_gemm_rows instance a fused call with M > 32 runs, if any: 32 rows x
 // one tile (kRowsT), 32 rows x two tiles (kRowsA) or 128 rows x two tiles
 // (kRowsC) a workgroup.  Each takes about t0 + rounds * (a + b KS) us, rounds
-// the workgroups per CU (fitted on MI355X to KS = 8 .. 54, M = 40 .. 2048, within
-// 15 %); the quickest by that runs while 128-row workgroups fit the chip once
-// (twice for gate||up, whose alternative has no wide form) or 32-row ones three
-// times.  Beyond that the tile kernels, which read each operand once per tile
-// and not once per 64 columns, are level or ahead.  Measured, tile kernel ->
-// this (us): 2560 -> 2 x 6912 relu2 M = 64 / 128 / 256: 14.4 / 14.3 / 15.2 ->
-// 6.8 / 8.9 / 13.7, M = 512 (not taken) 21.6 / 24.3; 6912 -> 2560 M = 64 / 128 /
-// 256 / 512 / 768: 19.2 / 20.2 / 20.1 / 21.3 / 23.1 -> 5.2 / 6.7 / 10.4 / 14.4 /
-// 18.3, M = 1024 (not taken) 26.8 / 31.3; 2560 -> 3840 M = 128 / 256 / 512: 15.1 /
-// 10.9 / 11.9 -> 4.5 / 6.2 / 9.6; 640 -> 160 M = 40 .. 2048: 6.6 .. 4.9 -> 3.2 .. 3.7.
+// the workgroups per CU; where the operand exceeds an XCD's 4 MB L2, at least the time that
+// its reads take, once per column group (once per two where 128 rows share
+// one) at 10 TB/s.  Fitted on MI355X; the quickest by that runs, among those
+// that beat the tile kernels.  These read each operand once per tile and not
+// once per 64 columns, so a form stays out from the rounds on where it loses:
+// the 32-row forms past three, the 128-row form past one (two for gate||up,
+// which has no wide form, up to 768 rows and from K = 1536).  From 1024
+// rows, where the tile kernels have many tiles: the 32-row forms past one (two tiles
+// and K > 1920: two), the 128-row form below K = 3969 and past 2048 rows.
+// Over 52 shapes (K 160 .. 16384, N 32 .. 32768) and 33 .. 4096 rows, 1200 points,
+// this is 0.4 % on average behind the best of the four, and behind the tile
+// kernels by more than 3 % at two (14336 -> 512 M = 1280 44.3 -> 46.8, 11008 -> 2 x 512
+// relu2 M = 1024 36.8 -> 39.0).  Measured with the prologue, tile kernel -> rows (us): 2560 -> 2 x
+// 6912 relu2 M = 64 / 128 / 256: 17.5 / 17.9 / 18.9 -> 10.2 / 12.7 / 18.4, M = 320 (not taken)
+// 24.2 -> 23.8; 6912 -> 2560 M = 64 / 128 / 256 / 512 / 768: 23.6 / 25.1 / 26.1 / 28.2 / 32.1 ->
+// 10.0 / 12.1 / 16.5 / 23.5 / 27.1, M = 1024 (not taken) 38.3 -> 41.0; 2560 -> 3840 M = 128 /
+// 256 / 512: 18.7 / 14.8 / 16.7 -> 8.6 / 10.5 / 14.8; 640 -> 160 M = 40 .. 2048: 9.6 .. 9.7 ->
+// 6.3 .. 9.3.  Not taken and why the lines: 12288 -> 1024 M = 2048 in 32 rows 63.9 -> 83.4, in 128
+// rows (taken) 59.5; 4096 -> 2 x 1024 relu2 M = 1536 29.1 -> 39.2; 256 -> 512 M = 4096 10.4 ->
+// 12.2.
 enum RowsKind { kRowsNone, kRowsT, kRowsA, kRowsC };
 static RowsKind rows_plan(int64_t M, int64_t K, int64_t N, int epilogue) {
   const int64_t Mb = mblocks(M), NT = N / 32, KS = ksb(K), cus = device_cus();
@@ -1762,12 +1772,19 @@ static RowsKind rows_plan(int64_t M, int64_t K, int64_t N, int epilogue) {
   auto rounds = [&](int64_t wgs) { return (wgs + cus - 1) / cus; };
   const int64_t pairs = relu2 ? NT / 2 : (NT + 1) / 2;
   const int64_t nt = rounds(NT * Mb), na = rounds(pairs * Mb), nc = rounds(pairs * ((Mb + 3) / 4));
-  if (nc > (relu2 ? 2 : 1) && na > 3) return kRowsNone;
-  const double tt = 2.2 + (double)nt * (0.65 + 0.045 * (double)KS);
-  const double ta = 2.4 + (double)na * (0.9 + 0.055 * (double)KS);
-  const double tc = 3.2 + (double)nc * (1.3 + 0.24 * (double)KS);
-  if (!relu2 && tt <= ta && tt <= tc) return kRowsT;
-  return ta <= tc ? kRowsA : kRowsC;
+  const bool many = M > 1024;
+  const bool t_ok = !relu2 && nt <= (many ? 1 : 3);
+  const bool a_ok = na <= (!many ? 3 : KS >= 16 ? 2 : 1);
+  const bool c_ok = many ? nc <= 1 && KS >= 32 && M <= 2048 : nc <= (relu2 && KS >= 12 && M <= 768 ? 2 : 1);
+  const int64_t operand = Mb * 32 * KS * 128;
+  const double reads = operand > 4000000 ? (double)operand / 1e7 : 0.0;  // us a pass
+  const double never = 1e30;
+  const double tt = t_ok ? 2.2 + std::max((double)nt * (0.65 + 0.045 * (double)KS), (double)NT * reads) : never;
+  const double ta = a_ok ? 2.4 + std::max((double)na * (0.9 + 0.055 * (double)KS), (double)pairs * reads) : never;
+  const double tc = c_ok ? 3.2 + std::max((double)nc * (1.3 + 0.24 * (double)KS), 0.5 * (double)pairs * reads) : never;
+  const double best = std::min({tt, ta, tc});
+  if (best == never) return kRowsNone;
+  return best == tt ? kRowsT : best == ta ? kRowsA : kRowsC;
 }
 
 template <int RBW, int RH, int TPW, int D, int EPI>
@@ -2025,6 +2042,11 @@ int btl_gemm_tiling(int64_t M, int64_t K, int64_t N, int epilogue, int rowsum_gi
     info[0] = 1, info[1] = g.rb * 32, info[2] = kPfCT, info[3] = rowsum_given ? g.splitk : 1;
   }
   return BTL_OK;
+}
+
+int btl_fused_prefill_form(int64_t M, int64_t K, int64_t N, int epilogue) {
+  if (M <= 0 || K <= 0 || N <= 0 || N % 32) return 0;
+  return rows_plan(M, K, N, epilogue);
 }
 
 int btl_choose_splitk(int64_t M, int64_t K, int64_t N, int epilogue) {

@@ -98,6 +98,11 @@ int btl_choose_splitk(int64_t M, int64_t K, int64_t N, int epilogue);
  * wide tiles store accumulators 16 bytes at a time, so a call with an acc_out
  * aligned to 4 bytes only runs the kind-1 tiles instead. */
 int btl_gemm_tiling(int64_t M, int64_t K, int64_t N, int epilogue, int rowsum_given, int32_t* info);
+/* The form of the GEMM that btl_bitlinear_fused runs for M > 32 (a planning
+ * query): 0 btl_gemm_i8t2's tiles (btl_gemm_tiling with row sums), else
+ * workgroups of 1: 32 rows x one column tile, 2: 32 rows x two, 3: 128 rows x
+ * two.  0 for M <= 32. */
+int btl_fused_prefill_form(int64_t M, int64_t K, int64_t N, int epilogue);
 int64_t btl_gemm_workspace_bytes(int64_t M, int64_t K, int64_t N, int epilogue, int splitk);
 int64_t btl_fused_workspace_bytes(int64_t M, int64_t K, int64_t N, int epilogue, int splitk);
 

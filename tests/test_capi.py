@@ -110,6 +110,28 @@ def test_gemm_tiling_invariants():
                 assert tiles <= 2 * 256, t
 
 
+def test_fused_prefill_form(L):
+    """The form a fused call with M > 32 runs, each side of the lines that the
+    rule draws: rounds of workgroups, operands larger than an L2 (a form with
+    fewer passes over them), and 1024 rows."""
+    f = L.btl_fused_prefill_form
+    T, A, C = 1, 2, 3
+    assert f(32, 2560, 2560, 0) == 0 and f(33, 2560, 2560, 0) == T and f(33, 2560, 33, 0) == 0
+    assert f(96, 2560, 3840, 0) == A and f(512, 2560, 3840, 0) == C and f(640, 2560, 3840, 0) == 0
+    assert f(768, 6912, 2560, 0) == C and f(896, 6912, 2560, 0) == 0
+    assert f(64, 2560, 13824, 1) == A and f(128, 2560, 13824, 1) == C
+    assert f(256, 2560, 13824, 1) == C and f(257, 2560, 13824, 1) == 0
+    # two rounds of 128 rows: not with a short K
+    assert f(192, 320, 12800, 1) == 0 and f(96, 640, 25600, 1) == 0
+    # an operand of 4 MB and more is read once per column group
+    assert f(512, 12288, 1024, 0) == A and f(2048, 12288, 1024, 0) == C and f(2049, 12288, 1024, 0) == 0
+    assert f(1024, 16384, 2048, 0) == C
+    # past 1024 rows: one round of 32 rows (two from K = 1921), one of 128 rows from K = 3969
+    assert f(2048, 640, 160, 0) in (T, A) and f(3072, 640, 160, 0) == 0
+    assert f(2048, 256, 512, 0) == 0 and f(1280, 2560, 640, 0) == A and f(2048, 2560, 640, 0) == 0
+    assert f(1536, 4096, 2048, 1) == 0 and f(2048, 1024, 2048, 1) == 0 and f(2048, 512, 256, 1) == A
+
+
 FAKE = 0x100000  # never dereferenced: every call below is rejected first
 
 

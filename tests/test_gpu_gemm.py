@@ -664,6 +664,9 @@ FEW_ROWS_SHAPES = [  # m, k, n, relu2
     (300, 160, 1056, False), (767, 6912, 2560, False), (769, 1056, 2560, False), (2048, 640, 160, False),
     (40, 64, 64, True), (64, 2560, 13824, True), (97, 2560, 13824, True), (250, 2560, 13824, True),
     (130, 992, 2112, True), (513, 1536, 8192, True), (257, 2560, 13824, True), (1000, 256, 1024, True),
+    # past 1024 rows: one round of one and of two tiles, two rounds, 128-row groups; an operand larger than an L2
+    (1500, 640, 160, False), (1793, 512, 256, True), (1300, 2560, 640, False), (1100, 4096, 1440, False),
+    (700, 12288, 1024, False),
 ]
 
 
