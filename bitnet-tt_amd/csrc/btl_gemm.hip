@@ -1518,6 +1518,9 @@ static GemmPlan plan_fused(int64_t M, int64_t K, int64_t N, int epilogue, int sp
   return pl;
 }
 
+enum RowsKind { kRowsNone, kRowsT, kRowsA, kRowsC };
+static RowsKind rows_plan(int64_t M, int64_t K, int64_t N, int epilogue);
+
 FusedLayout fused_layout(int64_t M, int64_t K, int64_t N, int epilogue, int splitk_req) {
   FusedLayout L;
   const int64_t rows = mblocks(M) * 32;
@@ -1525,9 +1528,12 @@ FusedLayout fused_layout(int64_t M, int64_t K, int64_t N, int epilogue, int spli
   L.a_dq = L.xa + round_up(btl_act_bytes(M, K), 256);
   L.rowsum = L.a_dq + round_up(rows * 4, 256);
   L.gemm_ws = L.rowsum + round_up(rows * 4, 256);
-  const GemmPlan pf = plan_fused(M, K, N, epilogue, splitk_req);
-  const GemmPlan pg = plan_gemm(M, K, N, epilogue, splitk_req);
-  L.total = L.gemm_ws + (pf.ws_bytes > pg.ws_bytes ? pf.ws_bytes : pg.ws_bytes);
+  L.total = L.gemm_ws;
+  if (rows_plan(M, K, N, epilogue) == kRowsNone) {  // the few-row workgroups need no partials or counters
+    const GemmPlan pf = plan_fused(M, K, N, epilogue, splitk_req);
+    const GemmPlan pg = plan_gemm(M, K, N, epilogue, splitk_req);
+    L.total += std::max(pf.ws_bytes, pg.ws_bytes);
+  }
   return L;
 }
 
@@ -1764,7 +1770,6 @@ static void launch_prefill_epi(bool prs, int rb, bool sk, dim3 grid, hipStream_t
 // 6.3 .. 9.3.  Not taken and why the lines: 12288 -> 1024 M = 2048 in 32 rows 63.9 -> 83.4, in 128
 // rows (taken) 59.5; 4096 -> 2 x 1024 relu2 M = 1536 29.1 -> 39.2; 256 -> 512 M = 4096 10.4 ->
 // 12.2.
-enum RowsKind { kRowsNone, kRowsT, kRowsA, kRowsC };
 static RowsKind rows_plan(int64_t M, int64_t K, int64_t N, int epilogue) {
   const int64_t Mb = mblocks(M), NT = N / 32, KS = ksb(K), cus = device_cus();
   const bool relu2 = epilogue == BTL_EPI_RELU2_MUL;

@@ -132,6 +132,18 @@ def test_fused_prefill_form(L):
     assert f(1536, 4096, 2048, 1) == 0 and f(2048, 1024, 2048, 1) == 0 and f(2048, 512, 256, 1) == A
 
 
+def test_fused_workspace_follows_the_form(L):
+    """A call that runs the few-row workgroups asks for no split-K partials,
+    so short prompts fit the static scratch; the tile kernels' calls still do."""
+    for m, k, n, epi in ((64, 6912, 2560, 0), (100, 6912, 2560, 0), (511, 2560, 3840, 0), (100, 2560, 13824, 1)):
+        assert L.btl_fused_prefill_form(m, k, n, epi) != 0 and L.btl_gemm_workspace_bytes(m, k, n, epi, 0) > 0
+        assert L.btl_fused_workspace_bytes(m, k, n, epi, 0) < L.btl_act_bytes(m, k) + (1 << 16)
+    m, k, n = 49 * 32, 16384, 39 * 32
+    assert L.btl_fused_prefill_form(m, k, n, 0) == 0
+    part = L.btl_gemm_workspace_bytes(m, k, n, 0, 0)
+    assert part > 0 and L.btl_fused_workspace_bytes(m, k, n, 0, 0) > L.btl_act_bytes(m, k) + part
+
+
 FAKE = 0x100000  # never dereferenced: every call below is rejected first
 
 

@@ -118,6 +118,8 @@ def test_noalloc_matches_workspace_entry_point(orc):
         (16, 2560, 2560, [0.02], [2560], N.EPI_SCALE, True),
         (32, 2560, 13824, [0.021, 0.018], [6912, 13824], N.EPI_RELU2_MUL, False),
         (64, 1024, 512, [0.02], [512], N.EPI_SCALE, True),
+        # a short prompt whose tile kernels would need 5 MiB of partials, its few-row workgroups none
+        (64, 6912, 2560, [0.02], [2560], N.EPI_SCALE, True),
     ]
     for i, (m, k, n, scales, ends, epi, with_res) in enumerate(cases):
         print(f"noalloc case {i}: m={m} k={k} n={n} epi={epi} residual={with_res}", flush=True)
