@@ -654,30 +654,35 @@ def test_cu_masked_stream_coresidency(orc):
         hip.hipStreamDestroy(raw)
 
 
-# Shapes of the short-prompt workgroups (M > 32 through the fused entry): 32
-# rows x 1 tile, 32 x 2 and 128 x 2, each with a ragged last row group, an odd
-# tile count, K not a multiple of 128, fewer superblocks than waves, and the
-# first shapes past the line where the tile kernels take over.
-FEW_ROWS_SHAPES = [  # m, k, n, relu2
-    (33, 32, 32, False), (33, 2560, 96, False), (64, 2560, 2560, False), (100, 2560, 2560, False),
-    (100, 6912, 2560, False), (129, 992, 3872, False), (256, 2560, 3840, False), (511, 2560, 3840, False),
-    (300, 160, 1056, False), (767, 6912, 2560, False), (769, 1056, 2560, False), (2048, 640, 160, False),
-    (40, 64, 64, True), (64, 2560, 13824, True), (97, 2560, 13824, True), (250, 2560, 13824, True),
-    (130, 992, 2112, True), (513, 1536, 8192, True), (257, 2560, 13824, True), (1000, 256, 1024, True),
+# Shapes of the short-prompt workgroups (M > 32 through the fused entry), with
+# the form each runs (btl_fused_prefill_form): 32 rows x 1 tile (1), 32 x 2 (2) and
+# 128 x 2 (3), each with a ragged last row group, an odd tile count, K not a
+# multiple of 128, fewer superblocks than waves; the first shapes past the lines
+# where the tile kernels (0) take over, one of them with split-K.
+FEW_ROWS_SHAPES = [  # m, k, n, relu2, form
+    (33, 32, 32, False, 1), (33, 2560, 96, False, 1), (64, 2560, 2560, False, 1), (100, 2560, 2560, False, 2),
+    (100, 6912, 2560, False, 2), (129, 992, 3872, False, 2), (256, 2560, 3840, False, 2), (511, 2560, 3840, False, 3),
+    (300, 160, 1056, False, 2), (767, 6912, 2560, False, 3), (769, 1056, 2560, False, 0), (2048, 640, 160, False, 2),
+    (40, 64, 64, True, 2), (64, 2560, 13824, True, 2), (97, 2560, 13824, True, 3), (250, 2560, 13824, True, 3),
+    (130, 992, 2112, True, 2), (513, 1536, 8192, True, 0), (257, 2560, 13824, True, 0), (1000, 256, 1024, True, 2),
     # past 1024 rows: one round of one and of two tiles, two rounds, 128-row groups; an operand larger than an L2
-    (1500, 640, 160, False), (1793, 512, 256, True), (1300, 2560, 640, False), (1100, 4096, 1440, False),
-    (700, 12288, 1024, False),
+    (1500, 640, 160, False, 1), (1793, 512, 256, True, 2), (1300, 2560, 640, False, 2), (1100, 4096, 1440, False, 3),
+    (700, 12288, 1024, False, 2),
+    # the tile kernels with split-K, whose counters the prologue clears
+    (1100, 2560, 1248, False, 0),
 ]
 
 
-@pytest.mark.parametrize("m,k,n,relu2", FEW_ROWS_SHAPES)
-def test_fused_few_rows_bit_exact(orc, m, k, n, relu2):
+@pytest.mark.parametrize("m,k,n,relu2,form", FEW_ROWS_SHAPES)
+def test_fused_few_rows_bit_exact(orc, m, k, n, relu2, form):
     """Quantised rows, accumulators and bf16 outputs of a fused call equal the
-    oracle's arithmetic, with a norm, three segments and an in-place residual
-    (scale) or two segments (relu2)."""
+    oracle's arithmetic in every row, with a norm, three segments and an
+    in-place residual (scale) or two segments (relu2); twice on the same
+    workspace.  The call runs the form that the shape is there for."""
     from bitnet_tt.ternary_matmul import PackedTernaryWeight, ternary_matmul_into
 
-    print(f"fused few rows m={m} k={k} n={n} relu2={relu2}", flush=True)
+    print(f"fused few rows m={m} k={k} n={n} relu2={relu2} form={form}", flush=True)
+    assert N.lib().btl_fused_prefill_form(m, k, n, int(relu2)) == form
     xb, gb = H.activations(orc, m, k, seed=m + 1), H.gamma(orc, k, seed=m + 2)
     w = H.ternary(k, n, seed=m + 3)
     if relu2 or n < 96:
@@ -688,26 +693,22 @@ def test_fused_few_rows_bit_exact(orc, m, k, n, relu2):
     scales = [0.013, 0.029, 0.021][: len(ends)]
     pw = PackedTernaryWeight(device_weight(orc, w), k, n, tuple(scales), tuple(ends))
     n_out = n // 2 if relu2 else n
-    out = torch.empty((m, n_out), dtype=torch.bfloat16, device=H.dev())
     res_bits = None
     if not relu2:
         res_bits = orc.f32_to_bf16(np.random.default_rng(m).standard_normal((m, n)).astype(np.float32))
-        out.copy_(H.to_dev_bf16(res_bits))
-    acc = torch.empty((m, n), dtype=torch.int32, device=H.dev())
-    xq = torch.empty((m, k), dtype=torch.int8, device=H.dev())
-    ternary_matmul_into(H.to_dev_bf16(xb), pw, out, norm_weight=H.to_dev_bf16(gb), norm_epsilon=1e-5,
-                        epilogue="relu2_mul" if relu2 else "none", residual=None if relu2 else out, acc_out=acc,
-                        xq_out=xq)
-    torch.cuda.synchronize()
-    rows = np.unique(np.concatenate([[0, 31, 32, m - 1], np.random.default_rng(k).integers(0, m, 6)]))
-    ref = orc.bitlinear(np.ascontiguousarray(xb[rows]), w, scales, ends, gamma_bf16=gb, norm_eps=1e-5)
-    q = xq.cpu().numpy()
-    assert np.array_equal(q[rows], ref["q"])
+    q, _, a_dq, _ = orc.act_quant_absmax(orc.bf16_to_f32(orc.rmsnorm_bf16(xb, gb, 1e-5, order=1)))
     full = full_acc_ref(orc, q, w, seed=m)
-    assert np.array_equal(acc.cpu().numpy(), full)
-    a_dq = np.zeros(m, np.float32)
-    a_dq[rows] = ref["a_dq"] if "a_dq" in ref else 0
-    got = H.bits_of(out)
-    exp = expected_out(orc, full[rows], a_dq[rows], scales, ends, int(relu2),
-                       None if res_bits is None else np.ascontiguousarray(res_bits[rows]))
-    assert np.array_equal(got[rows], exp)
+    exp = expected_out(orc, full, a_dq, scales, ends, int(relu2), res_bits)
+    x, g = H.to_dev_bf16(xb), H.to_dev_bf16(gb)
+    for rep in range(2):
+        out = torch.empty((m, n_out), dtype=torch.bfloat16, device=H.dev())
+        if res_bits is not None:
+            out.copy_(H.to_dev_bf16(res_bits))
+        acc = torch.empty((m, n), dtype=torch.int32, device=H.dev())
+        xq = torch.empty((m, k), dtype=torch.int8, device=H.dev())
+        ternary_matmul_into(x, pw, out, norm_weight=g, norm_epsilon=1e-5, epilogue="relu2_mul" if relu2 else "none",
+                            residual=None if relu2 else out, acc_out=acc, xq_out=xq)
+        torch.cuda.synchronize()
+        assert np.array_equal(xq.cpu().numpy(), q), rep
+        assert np.array_equal(acc.cpu().numpy(), full), rep
+        assert np.array_equal(H.bits_of(out), exp), rep
