@@ -243,10 +243,12 @@ template <bool EARLY>
 __device__ __forceinline__ bool att_load_first(AttnPair& a, const int32_t* pos, AttnRound& r) {
   const int wv = __builtin_amdgcn_readfirstlane(a.tid >> 6);
   // EARLY: the position is asked for ahead of the first blocks, and after
-  // everything that their loads need (the zero index depends on it): a wait
-  // for one scalar load is a wait for all.
-  int zero = 0;
-  if (EARLY) asm("s_mov_b32 %0, 0" : "=s"(zero) : "s"(a.kc), "s"(a.vc), "s"(a.S), "s"(a.Hkv));
+  // everything that their loads need (the index depends on it; the sign bits
+  // of sizes and addresses are zero): a wait for one scalar load is a wait for
+  // all.
+  const int zero = EARLY ? (int)(((uint32_t)(a.S | a.Hkv) >> 31) |
+                                 (uint32_t)((reinterpret_cast<uint64_t>(a.kc) | reinterpret_cast<uint64_t>(a.vc)) >> 63))
+                         : 0;
   const int apos = pos[zero];
   int blk = wv;
   bool any = true;
