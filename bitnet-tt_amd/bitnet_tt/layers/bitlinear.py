@@ -29,9 +29,8 @@ def quantize_and_transpose_weight(weight) -> tuple[np.ndarray, float]:
 def _device(device):
     import torch
 
-    if device is None:
-        return torch.device("cuda", torch.cuda.current_device())
-    return torch.device(device)
+    d = torch.device("cuda" if device is None else device)
+    return torch.device("cuda", torch.cuda.current_device()) if d.type == "cuda" and d.index is None else d
 
 
 def to_device_bf16(array, device):

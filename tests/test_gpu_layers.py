@@ -444,6 +444,24 @@ def test_c4_persistent_step_many_replays(orc, c4_model):
     assert not bad, f"replays {bad[:10]} differ from the oracle chain"
 
 
+@pytest.mark.parametrize("device", ["cuda", None, "cuda:0"])
+def test_load_weights_one_pass_however_the_device_is_named(orc, monkeypatch, device):
+    """A weight on the layer's device takes the one-pass load, also where the
+    device was given without an index; the same bytes as the host's."""
+    from bitnet_tt.layers import bitlinear as B
+
+    calls = []
+    real = B.quantize_for_gemm
+    monkeypatch.setattr(B, "quantize_for_gemm", lambda w: calls.append(1) or real(w))
+    w = (np.random.default_rng(11).standard_normal((96, 160)) * 0.02).astype(np.float32)
+    lin, ref = B.Linear(160, 96, device), B.Linear(160, 96, H.dev())
+    lin.load_weights(H.to_dev(w))
+    assert calls == [1]
+    ref.load_weights(w)
+    assert calls == [1] and lin.weight_scale == ref.weight_scale
+    assert torch.equal(lin.weight.data, ref.weight.data)
+
+
 def test_models_taking_turns_keep_their_own_step_workspace(orc):
     """Two models' one-launch steps in turn on one stream, with graph replays of
     the first between them, give what each gives alone; a model's workspaces
