@@ -9,6 +9,7 @@ calls are stream-ordered and can be recorded into a HIP graph.
 
 from __future__ import annotations
 
+import collections
 import ctypes
 import itertools
 import os
@@ -236,8 +237,19 @@ _workspaces: dict = {}
 # workspace_ptr's lookups: (kind, device index, stream, error offset, owner) ->
 # (address, bytes, buffer).  Emptied whenever a workspace is made or released.
 _fast: dict = {}
+# Held while the tables change or are read as a whole.  Not reentrant: a
+# finalizer may run inside (at any allocation) and must not change them then.
+_ws_lock = threading.Lock()
 _owner_ids = itertools.count(1)
 _owners: "weakref.WeakKeyDictionary" = weakref.WeakKeyDictionary()
+# Owners that went while the lock was held; released by the next workspace().
+_dead_owners: "collections.deque" = collections.deque()
+# Workspaces that went with unread error words: (key, buffer, offsets), read
+# and dropped by check_errors, or the oldest where a new one is made and there
+# are more than _RETIRED_MAX.  _late_errors: what the latter found.
+_retired: list = []
+_late_errors: list = []
+_RETIRED_MAX = 16
 
 
 def owner_id(obj) -> int:
@@ -251,13 +263,39 @@ def owner_id(obj) -> int:
 
 
 def _release_owner(n: int) -> None:
-    _fast.clear()
-    for key in [k for k in list(_workspaces) if len(k) == 4 and k[3] == n]:
-        buf = _workspaces.pop(key, None)
-        _error_words.pop(key, None)
-        if buf is not None:
-            _prepared_for.pop(buf.data_ptr(), None)
-            _reset_hooks.pop(buf.data_ptr(), None)
+    _dead_owners.append(n)
+    if _ws_lock.acquire(blocking=False):
+        try:
+            _bury()
+        finally:
+            _ws_lock.release()
+
+
+def _bury() -> None:
+    """Release the workspaces of the owners that are gone (lock held)."""
+    while _dead_owners:
+        n = _dead_owners.popleft()
+        _fast.clear()
+        for key in [k for k in _workspaces if len(k) == 4 and k[3] == n]:
+            _retire(key, _workspaces.pop(key))
+            _error_words.pop(key, None)
+
+
+def _retire(key, buf) -> None:
+    """A workspace that is replaced or released (lock held)."""
+    _prepared_for.pop(buf.data_ptr(), None)
+    _reset_hooks.pop(buf.data_ptr(), None)
+    offsets = sorted(_error_words.get(key, ()))
+    if offsets:
+        _retired.append((key, buf, offsets))
+
+
+def _set_words(key, buf, offsets) -> list:
+    """The error words of a workspace that are set: [(key, offset, value)]."""
+    import torch
+
+    words = [(key, off, int(buf[off:off + 4].view(torch.int32).item())) for off in offsets]
+    return [w for w in words if w[2]]
 
 
 def workspace_ptr(index: int, nbytes: int, kind: str, error_offset: int, stream: int, owner: int = 0):
@@ -268,8 +306,9 @@ def workspace_ptr(index: int, nbytes: int, kind: str, error_offset: int, stream:
     if hit is None or hit[1] < nbytes:
         import torch
 
-        buf = workspace(torch.device("cuda", index), nbytes, kind, error_offset, owner)
-        hit = _fast[key] = (buf.data_ptr(), buf.numel(), buf)
+        with _ws_lock:
+            buf = _workspace(torch.device("cuda", index), nbytes, kind, error_offset, owner)
+            hit = _fast[key] = (buf.data_ptr(), buf.numel(), buf)
     return hit
 
 
@@ -326,19 +365,30 @@ def workspace(device, nbytes: int, kind: str = "bitlinear", error_offset: int | 
     kind separates workspaces whose layouts differ ("bitlinear" for
     btl_bitlinear_fused / btl_gemm_i8t2, "step" for btl_decode_step).  A
     workspace that grows is replaced by a fresh zero-filled one; the old one
-    is released in stream order, after the calls that used it.
-    ``owner`` (owner_id) makes it one object's own.  ``error_offset`` registers the byte offset of a sticky error word inside
-    the workspace, which :func:`check_errors` reads."""
+    is released in stream order, after the calls that used it (one with an error
+    word once check_errors has read it).
+    ``owner`` (owner_id) makes it one object's own.  ``error_offset`` registers
+    the byte offset of a sticky error word inside the workspace, which
+    :func:`check_errors` reads."""
+    with _ws_lock:
+        return _workspace(device, nbytes, kind, error_offset, owner)
+
+
+def _workspace(device, nbytes: int, kind: str, error_offset: int | None, owner: int):
+    """workspace() with the lock held."""
     import torch
 
-    stream = torch.cuda.current_stream(device)
-    key = _key(kind, device, stream.cuda_stream, owner)
+    _bury()
+    key = _key(kind, device, torch.cuda.current_stream(device).cuda_stream, owner)
     buf = _workspaces.get(key)
     if buf is None or buf.numel() < nbytes:
         _fast.clear()
         if buf is not None:
-            _prepared_for.pop(buf.data_ptr(), None)
-            _reset_hooks.pop(buf.data_ptr(), None)
+            _retire(key, buf)
+        while len(_retired) > _RETIRED_MAX and not torch.cuda.is_current_stream_capturing():
+            old = _retired.pop(0)
+            torch.cuda.synchronize(old[0][1])
+            _late_errors.extend(_set_words(*old))
         size = max(int(nbytes), 1 << 20)
         buf = torch.zeros(size, dtype=torch.uint8, device=device)
         _prepared_for.pop(buf.data_ptr(), None)
@@ -366,27 +416,32 @@ def check_errors(device=None) -> None:
     import torch
 
     dev = _device_key(device if device is not None else "cuda")
-    keys = [k for k in _workspaces if k[1] == dev and _error_words.get(k)]
-    if not keys:
-        return
-    torch.cuda.synchronize(dev)
-    bad = []
-    for key in keys:
-        buf = _workspaces[key]
-        for off in sorted(_error_words[key]):
-            word = int(buf[off:off + 4].view(torch.int32).item())
-            if word:
-                bad.append((key, off, word))
+    with _ws_lock:
+        live = [(k, b, sorted(_error_words.get(k, ()))) for k, b in _workspaces.items() if k[1] == dev]
+        gone = [r for r in _retired if r[0][1] == dev]
+        _retired[:] = [r for r in _retired if r[0][1] != dev]
+        bad = [e for e in _late_errors if e[0][1] == dev]
+        _late_errors[:] = [e for e in _late_errors if e[0][1] != dev]
+    if gone or any(offsets for _, _, offsets in live):
+        torch.cuda.synchronize(dev)
+    for r in gone:
+        bad += _set_words(*r)
+    reset = []
+    for r in live:
+        found = _set_words(*r)
+        bad += found
+        if found:
+            reset.append(r[1])
     if not bad:
         return
-    for key in {b[0] for b in bad}:
-        _workspaces[key].zero_()
+    for buf in reset:
+        buf.zero_()
         torch.cuda.synchronize(dev)
-        hook = _reset_hooks.get(_workspaces[key].data_ptr())
+        hook = _reset_hooks.get(buf.data_ptr())
         if hook is not None:
             hook()
         else:
-            _prepared_for.pop(_workspaces[key].data_ptr(), None)
+            _prepared_for.pop(buf.data_ptr(), None)
     torch.cuda.synchronize(dev)
     what = ", ".join(f"{k[0]} workspace (stream {k[2]:#x}) word at byte {off} = {w}" for k, off, w in bad)
     raise RuntimeError(
