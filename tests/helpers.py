@@ -2,6 +2,7 @@
 configurations and bf16 bit-pattern transfers between numpy and torch."""
 
 import numpy as np
+import torch
 
 
 def dev():
@@ -204,3 +205,15 @@ def chain_agreement(orc, got_bits, ref_bits):
             "max_rel": float(np.abs(d).max() / np.abs(r).max()),
             "pcc": float(np.corrcoef(g.ravel(), r.ravel())[0, 1]),
             "bits_equal": float((np.asarray(got_bits) == np.asarray(ref_bits)).mean())}
+
+
+def step_workspace(step):
+    """The buffer that ``step``'s one-launch step runs on, on the current stream
+    (other models have their own)."""
+    from bitnet_tt import _native as N
+
+    ptr = step._step_workspace(attention=getattr(step, "kv", None) is not None)[0]
+    key = next(k for k in N._workspaces if k[0] == "step" and k[-1] == N.owner_id(step)
+               and k[2] == torch.cuda.current_stream().cuda_stream)
+    assert N._workspaces[key].data_ptr() == ptr
+    return N._workspaces[key]

@@ -330,8 +330,8 @@ def test_persistent_full_step_matches_step_full_2b(orc):
     # operand pieces, reads them and its weights again and redoes its MFMAs),
     # forced through the step workspace's test word: the attention instance's
     # own register allocation of that path gives the same bits.
-    key = next(k for k in N._workspaces if k[0] == "step" and k[2] == s.cuda_stream)
-    ws = N._workspaces[key]
+    with torch.cuda.stream(s):
+        ws = H.step_workspace(step)
     off = int(N.lib().btl_decode_step_error_offset()) + 64
     ws[off:off + 4] = torch.tensor([1, 0, 0, 0], dtype=torch.uint8, device=ws.device)
     try:
@@ -350,8 +350,7 @@ def test_persistent_full_step_matches_step_full_2b(orc):
 # (users, query heads, kv heads, cache length, positions): the edges of one
 # round (511..513 cached positions), of the blocks of 64, of the splits'
 # ranges and of the contexts that stay whole (896 and 1280 positions at 13 and 20
-# users); 8, 5, 3, 2 and 1 splits per pair; an out-of-range user among split ones
-# is left to test_position_out_of_range_is_flagged's single-split shape.
+# users); 8, 5, 3, 2 and 1 splits per pair.
 SPLIT_SHAPES = [
     (1, 4, 1, 4096, [4095]),
     (4, 20, 5, 4096, [0, 511, 512, 4095]),
@@ -373,6 +372,79 @@ def test_split_contexts(orc, B, Hq, Hkv, S, pos):
         att, cache, got, ref, kc, vc, kc2, vc2 = run(orc, B, Hq, Hkv, S, pos, seed == 52, seed)
         att.check()
         check(orc, got, ref, cache, kc2, vc2)
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,S,pos", [SPLIT_SHAPES[1], SPLIT_SHAPES[2], (4, 20, 5, 4096, [4095, -1, 4096, 700])])
+def test_split_contexts_around_bad_rows(orc, B, Hq, Hkv, S, pos):
+    """Cache rows past each user's position hold NaN and infinities, which
+    nothing of the output may take up (another split reads the row that split
+    0 writes); users outside the range among split ones give zeros, leave
+    their caches as they are and are flagged, and the same call with every
+    user in range is right after it."""
+    print(f"split attention, bad rows B={B} Hq={Hq} Hkv={Hkv} S={S}", flush=True)
+    rng = np.random.default_rng(57)
+    D = 128
+    qkv = orc.f32_to_bf16(rng.standard_normal((B, (Hq + 2 * Hkv) * D)).astype(np.float32))
+    kv = [orc.f32_to_bf16(rng.standard_normal((B, Hkv, S, D)).astype(np.float32)) for _ in "kv"]
+    bad = [p < 0 or p >= S for p in pos]
+    for c in kv:
+        for b, p in enumerate(pos):
+            c[b, :, max(p, 0):, 0::2] = 0x7FC0  # NaN
+            c[b, :, max(p, 0):, 1::2] = 0xFF80  # -inf
+    att = DecodeAttention(Hq, Hkv, D, S, H.dev())
+    cache = att.new_cache(B)
+    assert cache.split is not None
+    cache.key_cache.copy_(H.to_dev_bf16(kv[0]).view(B, Hkv, S, D))
+    cache.value_cache.copy_(H.to_dev_bf16(kv[1]).view(B, Hkv, S, D))
+    x = H.to_dev_bf16(qkv)
+    cos, sin = orc.rope_tables(D, S, 500000.0)
+    cur = list(pos)
+    for rep in range(2):
+        got = orc.bf16_to_f32(H.bits_of(att(x, cache, torch.tensor(cur, dtype=torch.int32, device=H.dev()))))
+        if rep == 0 and any(bad):
+            with pytest.raises(RuntimeError, match="out of range"):
+                att.check()
+        else:
+            att.check()
+        for b in range(B):
+            if rep == 0 and bad[b]:
+                assert not got[b].any()
+                assert np.array_equal(H.bits_of(cache.key_cache[b]).reshape(Hkv, S, D), kv[0][b])
+                assert np.array_equal(H.bits_of(cache.value_cache[b]).reshape(Hkv, S, D), kv[1][b])
+                continue
+            ref = orc.decode_attention(qkv[b:b + 1], kv[0][b:b + 1], kv[1][b:b + 1], np.asarray(cur[b:b + 1]), Hq, Hkv,
+                                       cos, sin, False, att.scale)[0]
+            tol = 2.0 ** -7 * np.abs(ref) + 1e-3 * np.abs(ref).max()
+            assert np.all(np.abs(got[b] - ref) <= tol), b
+        # the users that were outside: at the start of their cache
+        cur = [0 if f else p for f, p in zip(bad, pos)]
+
+
+def test_split_step_with_a_position_out_of_range(orc):
+    """The one-launch step with split contexts and one user outside the range:
+    the others' layer as step_full's, that user's attention zero, flagged; the
+    next step, every user in range, is right."""
+    from bitnet_tt.config import BitNet2B4TConfig
+    from bitnet_tt.decode import BitLinearDecodeStep
+
+    step = BitLinearDecodeStep.random_init(BitNet2B4TConfig(), H.dev(), seed=89, batch=5, num_layers=1)
+    step.alloc_buffers(seed=90).alloc_attention(max_seq_len=4096)
+    for pos in ([4095, 4096, 900, 64, 3000], [-1, 2000, 4095, 600, 513], [4095, 4000, 900, 64, 3000]):
+        step.pos.copy_(torch.tensor(pos, dtype=torch.int32))
+        bad = [b for b, p in enumerate(pos) if p < 0 or p >= 4096]
+        state = _full_state(step)
+        outs = []
+        for run_step in (step.step_full, step.step_persistent_full):
+            _restore(step, state)
+            run_step()
+            if bad:
+                with pytest.raises(RuntimeError, match="out of range"):
+                    step.check()
+            step.check()
+            outs.append(_outputs(step))
+        _compare(outs[1], outs[0], f"positions {pos}")
+        attn = step.attn_out.float()
+        assert all(bool((attn[b] == 0).all()) for b in bad)
 
 
 def test_whole_context_entry_needs_one_zero_word(orc):

@@ -397,8 +397,7 @@ def test_c4_persistent_step_reread_path(orc, c4_model):
     step.reset_hidden()
     step.step_persistent()  # prepares this stream's step workspace
     step.check()
-    key = next(k for k in N._workspaces if k[0] == "step" and k[2] == torch.cuda.current_stream().cuda_stream)
-    ws = N._workspaces[key]
+    ws = H.step_workspace(step)
     off = int(N.lib().btl_decode_step_error_offset()) + 64
     ws[off:off + 4] = torch.tensor([1, 0, 0, 0], dtype=torch.uint8, device=ws.device)
     try:
