@@ -149,9 +149,9 @@ def _segments(scales, ends):
     """segments_arrays of a weight's segments, kept by their values: a scale
     may be any object that converts to a float (a tensor or array may change
     in place between calls).  Zeros are not kept: 0.0 and -0.0 are equal keys."""
-    scales = tuple(map(float, scales))
-    ends = tuple(map(int, ends))
-    return N.segments_arrays(scales, ends) if 0.0 in scales else _cached_segments(scales, ends)
+    if type(sum(scales) + sum(ends)) is not float or 0.0 in scales:  # not plain numbers
+        return N.segments_arrays(scales, ends)
+    return _cached_segments(tuple(scales), tuple(ends))
 
 
 @functools.lru_cache(maxsize=4096)
@@ -237,7 +237,8 @@ def ternary_matmul_into(
         sc, en, nseg = N.segments_arrays(scales, tuple(w.segment_ends))
     index = x.device.index
     stream = N.raw_stream(index)
-    splitk = int(splitk)
+    if type(splitk) is not int:
+        splitk = int(splitk)
     nbytes, off = _fused_bytes(index, M, K, Nf, epi, splitk)
     ws, ws_bytes, _ = N.workspace_ptr(index, nbytes, "bitlinear", off, stream)
     rc = N.lib().btl_bitlinear_fused(x.data_ptr(), M, K, K, gamma, eps, w.data.data_ptr(), Nf, sc, en, nseg, epi, res,
