@@ -1771,9 +1771,9 @@ static void launch_prefill_epi(bool prs, int rb, bool sk, dim3 grid, hipStream_t
 // rows (taken) 59.5; 4096 -> 2 x 1024 relu2 M = 1536 29.1 -> 39.2; 256 -> 512 M = 4096 10.4 ->
 // 12.2.
 static RowsKind rows_plan(int64_t M, int64_t K, int64_t N, int epilogue) {
+  if (M <= 32 || M > (1 << 15)) return kRowsNone;
   const int64_t Mb = mblocks(M), NT = N / 32, KS = ksb(K), cus = device_cus();
   const bool relu2 = epilogue == BTL_EPI_RELU2_MUL;
-  if (M <= 32 || M > (1 << 15)) return kRowsNone;
   auto rounds = [&](int64_t wgs) { return (wgs + cus - 1) / cus; };
   const int64_t pairs = relu2 ? NT / 2 : (NT + 1) / 2;
   const int64_t nt = rounds(NT * Mb), na = rounds(pairs * Mb), nc = rounds(pairs * ((Mb + 3) / 4));
