@@ -19,8 +19,9 @@
 // (max, sum, unnormalised output per head) meet in one of them in a fixed
 // order.  One pair per workgroup leaves most of the chip idle there and walks
 // the rounds one after another: two users at 4096 positions, 5 key-value
-// heads, 48 us on 10 workgroups.  The number of splits depends on the pairs,
-// the cache length and the position only, so both callers give the same bits.
+// heads, 48 us on 10 workgroups.  The number of splits depends on the users,
+// the heads, the cache length and the position only (att_splits), so both
+// callers give the same bits.
 //  - Scores: v_mfma_f32_16x16x32_bf16, the G rotated query rows (head g at
 //    row 4 g, the other rows zero) against 16 cached key rows per MFMA (keys
 //    contiguous along D, the contraction, so the B operands load straight
