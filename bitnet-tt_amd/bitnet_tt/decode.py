@@ -259,6 +259,8 @@ class BitLinearDecodeStep:
         self.attn_out = acts(qd)
         self.qkv_out = torch.empty((B, c.qkv_dim), dtype=torch.bfloat16, device=self.device)
         self.ffn_h = torch.empty((B, c.intermediate_size), dtype=torch.bfloat16, device=self.device)
+        if not self.hidden.is_cuda:
+            return self
         # the one-launch step's workspace on this stream, with the buffers and
         # not in the first step (0 bytes: a shape that only step_per_call takes)
         L = N.lib()

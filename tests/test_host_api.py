@@ -147,3 +147,17 @@ def test_config_dims(known):
     assert (m.hidden_size, m.num_layers, m.num_attention_heads) == (256, 4, 4)
     with pytest.raises(ValueError):
         cfg.get_config("nope")
+
+
+def test_step_buffers_and_caches_on_the_cpu():
+    """A step's buffers and its KV caches can be made on the CPU (to be filled
+    or inspected there): they need neither the GPU nor its workspaces."""
+    torch = pytest.importorskip("torch")
+    from bitnet_tt.config import BitNetMiniConfig
+    from bitnet_tt.decode import BitLinearDecodeStep
+
+    step = BitLinearDecodeStep(BitNetMiniConfig(num_layers=2, num_attention_heads=2), torch.device("cpu"), batch=3)
+    step.layers = [None, None]
+    step.alloc_buffers(seed=5).alloc_attention(max_seq_len=1024)
+    assert step.hidden.shape == (3, step.config.hidden_size) and torch.equal(step.hidden, step.hidden0)
+    assert len(step.kv) == 2 and step.kv[0].key_cache.shape[2] == 1024 and step.pos.tolist() == [1023] * 3
