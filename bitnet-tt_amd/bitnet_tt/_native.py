@@ -214,8 +214,9 @@ def raw_stream(index: int) -> int:
 def stream_of(device) -> ctypes.c_void_p:
     import torch
 
-    d = torch.device(device)
-    return ctypes.c_void_p(raw_stream(torch.cuda.current_device() if d.index is None else d.index))
+    if isinstance(device, torch.device) and device.type == "cuda" and device.index is not None:
+        return ctypes.c_void_p(raw_stream(device.index))
+    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
 
 
 def segments_arrays(scales, ends):

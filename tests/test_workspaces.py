@@ -120,3 +120,24 @@ def test_growth_against_a_lookup(monkeypatch):
     hit = N.workspace_ptr(0, 64, "bitlinear", 16, 7)
     assert hit[1] == 4 << 20 and hit[0] != old.data_ptr()
     assert hit[2] is N._workspaces[("bitlinear", "cuda:0", 7)]
+
+
+def test_stream_of_takes_what_current_stream_takes(monkeypatch):
+    """None and indexless devices mean the current device, as for
+    torch.cuda.current_stream; what that refuses is refused."""
+    seen = []
+
+    def current_stream(device=None):
+        if device is not None and torch.device(device).type != "cuda":
+            raise ValueError("not a GPU")
+        seen.append(device)
+        return types.SimpleNamespace(cuda_stream=9)
+
+    monkeypatch.setattr(torch.cuda, "current_stream", current_stream)
+    monkeypatch.setattr(N, "_raw_stream", lambda index: 100 + index)
+    for device in (None, "cuda", torch.device("cuda"), 0):
+        assert N.stream_of(device).value == 9
+    assert seen == [None, "cuda", torch.device("cuda"), 0]
+    assert N.stream_of(torch.device("cuda", 1)).value == 101
+    with pytest.raises(ValueError):
+        N.stream_of(torch.device("cpu"))
