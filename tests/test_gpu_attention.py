@@ -420,16 +420,20 @@ def test_split_contexts_around_bad_rows(orc, B, Hq, Hkv, S, pos):
         cur = [0 if f else p for f, p in zip(bad, pos)]
 
 
-def test_split_step_with_a_position_out_of_range(orc):
+@pytest.mark.parametrize("positions", [
+    ([4095, 4096, 900, 64, 3000], [-1, 2000, 4095, 600, 513], [4095, 4000, 900, 64, 3000]),
+    ([4096], [4000], [-1], [100]),  # one user: its own kernel
+])
+def test_split_step_with_a_position_out_of_range(orc, positions):
     """The one-launch step with split contexts and one user outside the range:
     the others' layer as step_full's, that user's attention zero, flagged; the
     next step, every user in range, is right."""
     from bitnet_tt.config import BitNet2B4TConfig
     from bitnet_tt.decode import BitLinearDecodeStep
 
-    step = BitLinearDecodeStep.random_init(BitNet2B4TConfig(), H.dev(), seed=89, batch=5, num_layers=1)
+    step = BitLinearDecodeStep.random_init(BitNet2B4TConfig(), H.dev(), seed=89, batch=len(positions[0]), num_layers=1)
     step.alloc_buffers(seed=90).alloc_attention(max_seq_len=4096)
-    for pos in ([4095, 4096, 900, 64, 3000], [-1, 2000, 4095, 600, 513], [4095, 4000, 900, 64, 3000]):
+    for pos in positions:
         step.pos.copy_(torch.tensor(pos, dtype=torch.int32))
         bad = [b for b, p in enumerate(pos) if p < 0 or p >= 4096]
         state = _full_state(step)
