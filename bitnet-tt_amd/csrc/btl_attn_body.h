@@ -212,8 +212,9 @@ __device__ __forceinline__ uint4 att_ld(__amdgpu_buffer_rsrc_t r, int voff, int 
 // 32 loads are issued before anything that follows.  Left to itself the
 // compiler put half of a later round's loads in the one-launch step behind
 // waits for its first keys (32 users, cache of 4096, us a layer at position
-// 2000 / 4000: 55.5 / 85.5 against 52.7 / 80.8; 24 users' standalone call at 4000
-// 60.2 against 58.1); with all 32 ahead its instances spill 3 to 9 registers.
+// 2000 / 4000: 55.5 / 85.5 against 52.7 / 80.8; the standalone call of 24 / 32 users
+// at 4000 60.0 / 67.9 against 58.1 / 65.3, and 0.1 us more at one round, 11.3 against
+// 11.4); with all 32 ahead its instances spill 3 to 9 registers.
 template <bool AHEAD = false>
 __device__ __forceinline__ void att_load_block(const AttnPair& a, int blk, AttnRound& r) {
   const int lane = a.tid & 63, r16 = lane & 15, grp = lane >> 4, base = blk * kAtPosWave;
